@@ -35,6 +35,17 @@ __device__ __forceinline__ void split3(float x, uint32_t& h, uint32_t& m, uint32
     l = __float_as_uint(r2) >> 16;
 }
 
+// the three bf16 parts of two floats a, b, each part's pair packed (a low, b high)
+__device__ __forceinline__ void split3_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+    const uint32_t ha = __float_as_uint(a) & 0xffff0000u, hb = __float_as_uint(b) & 0xffff0000u;
+    const float ra = a - __uint_as_float(ha), rb = b - __uint_as_float(hb);
+    const uint32_t ma = __float_as_uint(ra) & 0xffff0000u, mb = __float_as_uint(rb) & 0xffff0000u;
+    const float la = ra - __uint_as_float(ma), lb = rb - __uint_as_float(mb);
+    h = (ha >> 16) | hb;
+    m = (ma >> 16) | mb;
+    l = (__float_as_uint(la) >> 16) | (__float_as_uint(lb) & 0xffff0000u);
+}
+
 // Wave-wide reductions. Within each row of 16 lanes the partner values move by DPP (quad
 // xor 1, quad xor 2, half-row mirror, row mirror: after the four steps every lane holds its
 // row's total), the two rows of each half-wave meet through a swizzle (xor 16 within 32

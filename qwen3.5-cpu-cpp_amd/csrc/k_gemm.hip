@@ -75,18 +75,6 @@ constexpr int kFlush = 16;   // stages per partial sum (K = 512)
 constexpr int kLd = kBK + 16;  // padded W row in LDS (bf16 elements): 96 B
 constexpr int kCB = kBN / 16;  // 16-column MFMA blocks per wave (two 16-row blocks)
 
-// the three bf16 parts of two floats a, b, each part's pair packed (a low, b high)
-__device__ __forceinline__ void split3_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-    const uint32_t ha = __float_as_uint(a) & 0xffff0000u, hb = __float_as_uint(b) & 0xffff0000u;
-    const float ra = a - __uint_as_float(ha), rb = b - __uint_as_float(hb);
-    const uint32_t ma = __float_as_uint(ra) & 0xffff0000u, mb = __float_as_uint(rb) & 0xffff0000u;
-    const float la = ra - __uint_as_float(ma), lb = rb - __uint_as_float(mb);
-    h = (ha >> 16) | hb;
-    m = (ma >> 16) | mb;
-    l = (__float_as_uint(la) >> 16) | (__float_as_uint(lb) & 0xffff0000u);
-}
-
-// the two fp16 parts of two (scaled) floats a, b: h = rn(x), l = rn(x - h), each pair packed
 // One 128 x 128 tile. MASK: some W rows of the tile lie past N or K is not a whole number of
 // flush blocks, so W and X chunks past N or K are zeroed (X rows past M are clamped to row 0
 // and their outputs dropped).
@@ -380,12 +368,15 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
 
 }  // namespace
 
+// Few tokens go to k_gemm_small.hip where that is expected to be faster (its small_plan).
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
     dim3 grid(gemm_col_tiles(a.N), (a.M + kBM - 1) / kBM);
     const bool f16 = a.Wh && a.xmax && a.xmax_n > 0 && a.x_tiled && a.K % 32 == 0;
     // the tiled layouts exist on the two-part path only (Y: its SwiGLU output)
     if ((a.x_tiled && !f16) || (a.y_tiled && !(f16 && a.swiglu && (a.N / 2) % 32 == 0))) return hipErrorInvalidValue;
     if (a.x_planes && !(f16 && a.xmax_n == 1)) return hipErrorInvalidValue;  // the producer's one row maximum
+    hipError_t e = hipSuccess;
+    if (launch_gemm_small(a, s, &e)) return e;
     if (f16 && a.x_planes) {
         if (a.swiglu) klaunch(gemm_kernel<2, true, true>, grid, 256, 0, s, a);
         else if (a.R) klaunch(gemm_kernel<1, true, true>, grid, 256, 0, s, a);

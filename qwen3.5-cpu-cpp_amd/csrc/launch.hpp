@@ -98,8 +98,8 @@ struct GemmArgs {
     int w_exp = 0;
     const float* xmax = nullptr;
     int xmax_n = 0;
-    // SwiGLU output: the maximum |Y| of each row over each column tile (N / 128 wide rows:
-    // ymax[r * ceil(N / 128) + tile]) for the next GEMM's two-part path (may be null)
+    // SwiGLU output: the maximum |Y| of each row over each column tile, in rows of
+    // gemm_ymax_parts() of them, for the next GEMM's two-part path (may be null)
     float* ymax = nullptr;
     // X (two-part path) and, for SwiGLU, Y in the tiled layout of xt_off (ldx / ldy unused;
     // rows padded to a multiple of 128, K to a multiple of 32)
@@ -109,6 +109,14 @@ struct GemmArgs {
     int x_planes = 0;
 };
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t s);
+// The same results by the kernel for few tokens where it is expected to be faster (false: it
+// is not, nothing was launched). Called by launch_gemm, which has checked `a`.
+bool launch_gemm_small(const GemmArgs& a, hipStream_t s, hipError_t* e);
+// Partial maxima per row that launch_gemm(a) writes to a.ymax (a.ymax itself is not read),
+// and the most there can be for N columns of up to kGemmSmallRows rows
+int gemm_ymax_parts(const GemmArgs& a);
+constexpr int kGemmSmallRows = 1024;
+inline int gemm_small_max_parts(int N) { return N / 16 + 272; }
 // Tiled activation layout of the two-part GEMM's X operand: blocks of 16 rows x 32 k
 // (512 floats), row block after row block and within one the k blocks in order; inside a
 // block [h][r][g][e] for k = 8 g + 4 h + e of row r: the 16 bytes a lane of the matrix-core
@@ -128,7 +136,7 @@ __host__ __device__ inline int64_t xp_off(int64_t row, int k, int K, int part) {
     return ((row >> 4) * (K >> 5) + (k >> 5)) * 1024 + part * 512 + (((k & 31) >> 3) << 7) + ((row & 15) << 3) +
            (k & 7);
 }
-// Column tiles of the GEMM (the ymax row width)
+// Column tiles of the 128 x 128 GEMM
 inline int gemm_col_tiles(int N) { return (N + 127) / 128; }
 // max |w| over n bf16 weights, into *out (a uint zeroed beforehand: the bits of the
 // non-negative maximum); and wh = fp16(w x 2^e), round to nearest even

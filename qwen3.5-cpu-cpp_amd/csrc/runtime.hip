@@ -768,7 +768,8 @@ PrefillPlan plan_prefill(const q35_dims& d, int tb, int64_t logits_width, bool e
     p.ids = take(T);
     p.xn_max = take(T);
     p.mix_max = take(T * std::max(d.attn_q_heads, d.gdn_v_heads));
-    p.hb_max = take(T * q35k::gemm_col_tiles(2 * d.ffn_intermediate));
+    p.hb_max = take(std::max(T * q35k::gemm_col_tiles(2 * d.ffn_intermediate),
+                             std::min<int64_t>(T, q35k::kGemmSmallRows) * q35k::gemm_small_max_parts(2 * d.ffn_intermediate)));
     p.wmax = take(4LL * d.n_layers_total);
     if (p.tiled) {  // the fp16 weight copies of the two-part path
         int64_t wh = 0;
@@ -1104,10 +1105,12 @@ hipError_t gemm(const float* X, int64_t ldx, const uint16_t* W, int M, int N, in
 }
 
 // The same on the two-part fp16 path: weight matrix i of layer ly, the row maxima of X
-// (xmax_n partial maxima per row), and for the SwiGLU GEMM the row maxima of its output.
+// (xmax_n partial maxima per row), and for the SwiGLU GEMM the row maxima of its output
+// (ymax_parts of them per row).
 // tiled: 0 row-major X (three exact bf16 parts), 1 tiled fp32 X, 2 X split by its producer.
 hipError_t gemm_h(const float* X, int64_t ldx, const LayerDev& ly, int i, const float* xmax, int xmax_n, int M, int N,
-                  int K, const float* R, float* Y, int64_t ldy, hipStream_t s, int tiled, float* ymax = nullptr) {
+                  int K, const float* R, float* Y, int64_t ldy, hipStream_t s, int tiled, float* ymax = nullptr,
+                  int* ymax_parts = nullptr) {
     const uint16_t* W[4] = {ly.w_in, ly.w_out, ly.w_gu, ly.w_down};
     q35k::GemmArgs g{X, W[i], R, Y, M, N, K, ldx, R ? ldy : 0, ldy};
     g.swiglu = ymax != nullptr;
@@ -1119,6 +1122,7 @@ hipError_t gemm_h(const float* X, int64_t ldx, const LayerDev& ly, int i, const 
     g.x_tiled = tiled != 0;
     g.x_planes = tiled == 2;
     g.y_tiled = tiled && ymax != nullptr;
+    if (ymax_parts) *ymax_parts = q35k::gemm_ymax_parts(g);
     return q35k::launch_gemm(g, s);
 }
 
@@ -1211,9 +1215,10 @@ q35_status prefill_block(q35_model* m, const PrefillPlan& p, int pos0, int T, in
         });
         // gate/up projection with silu(gate) * up in its epilogue: hb = T x I, with the row
         // maxima of hb per column tile for the down projection
-        Lr.run(Q35_KT_GEMM, [&] { return gemm_h(xn, H, ly, 2, xn_max, 1, T, 2 * I, H, nullptr, hb, I, s, xn_form, hb_max); });
+        int hb_parts = 0;
+        Lr.run(Q35_KT_GEMM, [&] { return gemm_h(xn, H, ly, 2, xn_max, 1, T, 2 * I, H, nullptr, hb, I, s, xn_form, hb_max, &hb_parts); });
         Lr.run(Q35_KT_GEMM, [&] {
-            return gemm_h(hb, I, ly, 3, hb_max, q35k::gemm_col_tiles(2 * I), T, H, I, hidden, hidden, H, s, p.tiled);
+            return gemm_h(hb, I, ly, 3, hb_max, hb_parts, T, H, I, hidden, hidden, H, s, p.tiled);
         });
         if (trace_host)
             Lr.run(Q35_KT_OTHER, [&] {
