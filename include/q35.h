@@ -400,9 +400,12 @@ q35_status q35_gdn_prefill(const q35_gdn_prefill_args *args, q35_stream s);
  *   k_cache, v_cache [NKV][max_context][HD]; out [n][NQ * HD]
  * workspace (16-byte aligned): q35_attn_prefill_workspace_bytes() bytes. With an fp32 cache
  * that size includes the keys and values of positions [0, pos0 + n) pre-split into the
- * attention kernel's tile layout (3 KB per position and kv head); a workspace of at least
- * NQ * n * HD * 4 + 256 bytes but smaller than that is accepted, and the kernel then splits
- * every tile itself (slower, same results). Requires HD == 256. */
+ * attention kernel's tile layout (3 KB per position and kv head), and, for few tokens on
+ * more than 2048 positions, the partial outputs of key ranges that run in parallel (up to
+ * 135 MB). A workspace of at least NQ * n * HD * 4 + 256 bytes but smaller than that is
+ * accepted: without room for the tiles the kernel splits every tile itself (slower, same
+ * results), without room for the partial outputs it walks all keys of a block in one
+ * workgroup (slower, the same results to fp32 rounding). Requires HD == 256. */
 typedef struct q35_attn_prefill_args {
     int32_t n_tokens, pos0, q_heads, kv_heads, head_dim, rotary_dim;
     int32_t kv_dtype;      /* cache elements: 0 = fp32, 1 = bf16 (as q35_attn_decode_args) */

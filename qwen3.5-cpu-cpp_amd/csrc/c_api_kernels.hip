@@ -369,18 +369,28 @@ q35_status q35_gdn_prefill(const q35_gdn_prefill_args* args, q35_stream s) {
 }
 
 namespace {
-// without the pre-split key / value tiles (the least q35_attn_prefill accepts)
+// without the pre-split key / value tiles and the partial outputs (the least
+// q35_attn_prefill accepts)
 uint64_t attn_prefill_min_bytes(const q35_attn_prefill_args& g) {
     return static_cast<uint64_t>(q35k::attn_prefill_workspace_floats(g.q_heads, g.n_tokens)) * 4;
+}
+// the pre-split key / value tiles (fp32 cache)
+uint64_t attn_prefill_image_bytes(const q35_attn_prefill_args& g) {
+    return g.kv_dtype == 0 && g.kv_heads > 0 && g.pos0 >= 0
+               ? static_cast<uint64_t>(q35k::attn_prefill_image_floats(g.kv_heads, g.pos0, g.n_tokens)) * 4
+               : 0;
+}
+// partial outputs of the key ranges, where the kernel would split them
+int attn_prefill_slots(const q35_attn_prefill_args& g) {
+    if (g.kv_heads <= 0 || g.q_heads % g.kv_heads != 0 || g.pos0 < 0) return 0;
+    return q35k::flash_plan(g.n_tokens, g.q_heads, g.kv_heads, g.pos0, g.kv_dtype == 1).slots;
 }
 }  // namespace
 
 uint64_t q35_attn_prefill_workspace_bytes(const q35_attn_prefill_args* args) {
     if (!args || args->q_heads <= 0 || args->n_tokens <= 0) return 0;
-    uint64_t n = attn_prefill_min_bytes(*args);
-    if (args->kv_dtype == 0 && args->kv_heads > 0 && args->pos0 >= 0)
-        n += static_cast<uint64_t>(q35k::attn_prefill_image_floats(args->kv_heads, args->pos0, args->n_tokens)) * 4;
-    return n;
+    return attn_prefill_min_bytes(*args) + attn_prefill_image_bytes(*args) +
+           static_cast<uint64_t>(q35k::attn_prefill_part_floats(attn_prefill_slots(*args))) * 4;
 }
 
 q35_status q35_attn_prefill(const q35_attn_prefill_args* args, q35_stream s) {
@@ -422,8 +432,18 @@ q35_status q35_attn_prefill(const q35_attn_prefill_args* args, q35_stream s) {
     a.v_cache = g.v_cache;
     a.kv_bf16 = g.kv_dtype == 1;
     a.Qa = static_cast<float*>(g.workspace);
-    if (!a.kv_bf16 && g.workspace_bytes >= q35_attn_prefill_workspace_bytes(args))
-        a.kv_img = a.Qa + q35k::attn_prefill_workspace_floats(a.NQ, a.T);
+    // what the workspace has room for: the pre-split tiles first, then the partial outputs
+    uint64_t used = attn_prefill_min_bytes(g);
+    const uint64_t img = attn_prefill_image_bytes(g);
+    if (img && g.workspace_bytes >= used + img) {
+        a.kv_img = a.Qa + used / 4;
+        used += img;
+    }
+    const int slots = attn_prefill_slots(g);
+    if (slots && g.workspace_bytes >= used + static_cast<uint64_t>(q35k::attn_prefill_part_floats(slots)) * 4) {
+        a.part = a.Qa + used / 4;
+        a.part_slots = slots;
+    }
     a.out = g.out;
     return launched(q35k::launch_attn_prefill(a, as_stream(s)), "q35_attn_prefill");
 }

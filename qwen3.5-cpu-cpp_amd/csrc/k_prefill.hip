@@ -729,16 +729,30 @@ __global__ __launch_bounds__(256) void attn_prefill_prep_kernel(AttnPrefillArgs 
 }
 
 // ------------------------------------------------------------------ flash attention
-constexpr int kFW = 8;            // waves per workgroup
-constexpr int kQT = 16 * kFW;     // query rows per workgroup (16 per wave)
+// waves per workgroup, 16 query rows each: with a bf16 cache two workgroups of 4 share a
+// compute unit, and one's staging and barriers run under the other's products
+constexpr int kBf16Waves = 4;
+constexpr int flash_waves(bool kv_bf16) { return kv_bf16 ? kBf16Waves : 8; }
 constexpr int kKT = 32;           // keys per tile
+constexpr int kFlashPieces = 128;  // most pieces of a block
 constexpr float kLog2e = 1.44269504088896341f;
 
-// 128 query rows of one head per workgroup (16 per wave), causal, keys of earlier blocks from
-// the cache, 32-key tiles staged through LDS (the next tile's rows are loaded into registers
-// while the current one is multiplied), online softmax. One workgroup per CU (112 KB of LDS
-// with three parts); causal work grows with the query block, and workgroups are dispatched
-// in linear order, so block L takes the L-th longest item (query blocks from the last).
+// 128 query rows per workgroup (16 per wave), causal, keys of earlier blocks from the cache,
+// 32-key tiles staged through LDS (the next tile's rows are loaded into registers while the
+// current one is multiplied), online softmax. One workgroup per CU (112 KB of LDS with three
+// parts). A row is a (token, query head of the kv head's group) pair, row = token * group +
+// head: the heads of a group read the same keys, so 32 tokens of a group of 4 are one full
+// block and not four quarter ones, and a block's rows end within 128 / group tokens of each
+// other. Causal work grows with the block, and workgroups are dispatched in linear order, so
+// rank L takes the L-th longest block of all kv heads.
+//
+// Few blocks over many keys (a chat turn: 300 tokens of 2 x 4 heads are 20 blocks) would
+// leave most compute units idle, so a block's tiles are then cut into pieces of `piece`
+// tiles, one workgroup each (flash_plan), whose unnormalised outputs, maxima and sums
+// flash_combine_kernel merges. 300 tokens at 7000 cached bf16 positions, 8 / 2 heads: 24
+// blocks of single heads 703 us; 494 pieces 82 us (flash 74, of which about 8 the query rows
+// and the partial outputs; merge 12 for 32 MB of them). Bound as the unsplit kernel: products
+// behind LDS reads and two barriers a tile.
 // Both products run on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16): every fp32 operand
 // is the exact sum of three bf16 parts (hi + mid + lo, as in the bf16 path of the projection GEMM), and a
 // product a.b is the sum of the six part products a_i b_j with i + j <= 2 (parts counted
@@ -818,16 +832,25 @@ __global__ __launch_bounds__(256) void attn_kv_image_kernel(AttnPrefillArgs a) {
 }
 
 // IMG (fp32 cache only): tiles are copied from the image attn_kv_image_kernel wrote.
-template <bool KVB, bool IMG>
-__global__ __launch_bounds__(kFW * 64, 1) void flash_attn_kernel(AttnPrefillArgs a) {
+// SPLIT: grid (pieces, blocks of all kv heads), else grid (blocks).
+template <bool KVB, bool IMG, bool SPLIT>
+__global__ __launch_bounds__(flash_waves(KVB) * 64, KVB ? 8 / flash_waves(KVB) : 1) void flash_attn_kernel(AttnPrefillArgs a) {
     static_assert(!(KVB && IMG), "the tile image holds the parts of an fp32 cache");
+    constexpr int kFW = flash_waves(KVB), kQT = 16 * kFW;
+    constexpr int SS = 8 / kFW;  // staging passes (one thread's share of a tile by 512 threads each)
     constexpr int NP = KVB ? 1 : 3;  // parts of K and V
-    const int nqt = gridDim.x;
-    const int rank = blockIdx.x + blockIdx.y * nqt;
-    const int qt = nqt - 1 - rank / a.NQ, h = rank % a.NQ;
+    const int grp = a.NQ / a.NKV, rows = a.T * grp, nblk = (rows + kQT - 1) / kQT;
+    const int rank = SPLIT ? blockIdx.y : blockIdx.x;
+    const int qt = nblk - 1 - rank / a.NKV, kh = rank % a.NKV;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int grp = a.NQ / a.NKV, kh = h / grp;
-    const int t0 = qt * kQT;
+    const int row0 = qt * kQT;
+    // keys of the block, and this workgroup's piece of them
+    const int kv_end = a.pos0 + min(rows - 1, row0 + kQT - 1) / grp + 1;
+    const int piece_keys = a.piece * kKT;
+    const int kv_lo = SPLIT ? static_cast<int>(blockIdx.x) * piece_keys : 0;
+    if (SPLIT && kv_lo >= kv_end) return;  // uniform: the block has fewer pieces
+    const int kv_hi = SPLIT ? min(kv_end, kv_lo + piece_keys) : kv_end;
+    const bool whole = !SPLIT || kv_end <= piece_keys;  // the block's only piece: final output
     const int r16 = lane & 15, g4 = lane >> 4;
     // LDS in 16-byte chunks (8 bf16) so that the 16 lanes of a lane group read one whole
     // 256-byte row of 16 chunks (any order within the row runs at full rate; rows of padded
@@ -839,10 +862,10 @@ __global__ __launch_bounds__(kFW * 64, 1) void flash_attn_kernel(AttnPrefillArgs
     const float sc = 1.0f / sqrtf(static_cast<float>(kHD));
 
     // this lane's query row, dims 32c + 8 g4 .. + 7, as three bf16 parts (the B operand)
-    const int qrow = t0 + wave * 16 + r16;
+    const int qrow = min(row0 + wave * 16 + r16, rows - 1);
     bf16x8 qp[3][8];
     {
-        const float* src = a.Qa + (static_cast<int64_t>(h) * a.T + min(qrow, a.T - 1)) * kHD + 8 * g4;
+        const float* src = a.Qa + (static_cast<int64_t>(kh * grp + qrow % grp) * a.T + qrow / grp) * kHD + 8 * g4;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             const float4 x0 = *reinterpret_cast<const float4*>(src + 32 * c);
@@ -856,15 +879,14 @@ __global__ __launch_bounds__(kFW * 64, 1) void flash_attn_kernel(AttnPrefillArgs
                 qp[p][c] = __builtin_bit_cast(bf16x8, make_uint4(p0[p].x, p0[p].y, p1[p].x, p1[p].y));
         }
     }
-    const int qpos = a.pos0 + qrow;
+    const int qpos = a.pos0 + qrow / grp;
     // the wave's last query position: tiles starting past it hold no key its rows attend
-    const int wlast = a.pos0 + min(t0 + wave * 16 + 15, a.T - 1);
+    const int wlast = a.pos0 + min(row0 + wave * 16 + 15, rows - 1) / grp;
     floatx4 o[16];  // dims 16 t + r16 of query rows 4 g4 + v
 #pragma unroll
     for (int t = 0; t < 16; ++t) o[t] = floatx4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.0f;
 
-    const int kv_end = a.pos0 + min(a.T, t0 + kQT);
     const int64_t hoff = static_cast<int64_t>(kh) * a.max_ctx * kHD;
     // staging of one tile, in registers while the previous tile is multiplied: K key
     // 8 (wave % 4) + lane % 8, dim chunks 8 c + lane / 8 for c = 2 (wave / 4) + i, i < 2 (two
@@ -872,11 +894,16 @@ __global__ __launch_bounds__(kFW * 64, 1) void flash_attn_kernel(AttnPrefillArgs
     // 4 g .. + 3 and 16 + 4 g .. + 3, one float2 each); split (or widened) when stored to LDS
     const int ks_row = 8 * (wave & 3) + (lane & 7), ks_c0 = 16 * (wave >> 2) + (lane >> 3);
     const int vs_g = tid & 3, vs_d = (tid >> 2) * 2;
-    float4 kst[IMG ? 1 : 4];
-    float2 vst[IMG ? 1 : 8];
+    float4 kst[IMG || KVB ? 1 : 4];
+    float2 vst[IMG || KVB ? 1 : 8];
     // (vector-typed: an array of uint4 structs here was placed in scratch memory)
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     u32x4 ist[IMG ? kImgTile / (kFW * 64) : 1];
+    // bf16 cache: the stored bits are the operands, K chunks as they lie, V pairs of dims
+    // (8-byte aligned, as the cache rows' other accesses)
+    typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+    u32x4 kbs[KVB ? 2 * SS : 1];
+    uint32_t vbs[KVB ? 8 * SS : 1];
     auto vkey = [&](int j) { return vslot_key(vs_g, j); };
     auto load_tile = [&](int kv0) {
         if constexpr (IMG) {  // tiles past the block's keys: the last one again (in the image)
@@ -887,38 +914,31 @@ __global__ __launch_bounds__(kFW * 64, 1) void flash_attn_kernel(AttnPrefillArgs
             return;
         }
         const bool live = kv0 < kv_end;
+        if constexpr (KVB) {
+            const uint16_t *kc = reinterpret_cast<const uint16_t*>(a.k_cache) + hoff,
+                           *vc = reinterpret_cast<const uint16_t*>(a.v_cache) + hoff;
+            const int64_t ok = live ? static_cast<int64_t>(min(kv0 + ks_row, kv_end - 1)) * kHD : 0;
+#pragma unroll
+            for (int j = 0; j < 2 * SS; ++j) kbs[j] = *reinterpret_cast<const u32x4_a8*>(kc + ok + 8 * (ks_c0 + 8 * j));
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int64_t ov = live ? static_cast<int64_t>(min(kv0 + vkey(j), kv_end - 1)) * kHD + vs_d : 0;
+#pragma unroll
+                for (int e = 0; e < SS; ++e) vbs[8 * e + j] = *reinterpret_cast<const uint32_t*>(vc + ov + e * (kHD / SS));
+            }
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int pk = min(kv0 + ks_row, kv_end - 1);
             const int64_t ok = live ? static_cast<int64_t>(pk) * kHD + 8 * (ks_c0 + 8 * (j >> 1)) + 4 * (j & 1) : 0;
-            if constexpr (KVB) {
-                const uint2 kb = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(a.k_cache) + hoff + ok);
-                kst[j] = make_float4(bf16_lo(kb.x), bf16_hi(kb.x), bf16_lo(kb.y), bf16_hi(kb.y));
-            } else {
-                kst[j] = *reinterpret_cast<const float4*>(a.k_cache + hoff + ok);
-            }
+            kst[j] = *reinterpret_cast<const float4*>(a.k_cache + hoff + ok);
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int pv = min(kv0 + vkey(j), kv_end - 1);
             const int64_t ov = live ? static_cast<int64_t>(pv) * kHD + vs_d : 0;
-            if constexpr (KVB) {
-                const uint32_t vb = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(a.v_cache) + hoff + ov);
-                vst[j] = make_float2(bf16_lo(vb), bf16_hi(vb));
-            } else {
-                vst[j] = *reinterpret_cast<const float2*>(a.v_cache + hoff + ov);
-            }
-        }
-    };
-    // eight floats as NP 16-byte chunks: three exact bf16 parts, or (a bf16 cache) the values
-    auto parts8 = [&](const float (&x)[8], uint4 (&c)[NP]) {
-        if constexpr (KVB) {
-            c[0] = make_uint4(__float_as_uint(x[0]) >> 16 | (__float_as_uint(x[1]) & 0xffff0000u),
-                              __float_as_uint(x[2]) >> 16 | (__float_as_uint(x[3]) & 0xffff0000u),
-                              __float_as_uint(x[4]) >> 16 | (__float_as_uint(x[5]) & 0xffff0000u),
-                              __float_as_uint(x[6]) >> 16 | (__float_as_uint(x[7]) & 0xffff0000u));
-        } else {
-            split3_8(x, c);
+            vst[j] = *reinterpret_cast<const float2*>(a.v_cache + hoff + ov);
         }
     };
     // Rows past the end of the keys are copies of the last one (finite): their scores are
@@ -932,12 +952,33 @@ __global__ __launch_bounds__(kFW * 64, 1) void flash_attn_kernel(AttnPrefillArgs
             for (int j = 0; j < NJ / 2; ++j) reinterpret_cast<u32x4*>(&Vc[0][0][0][0])[tid + kFW * 64 * j] = ist[NJ / 2 + j];
             return;
         }
+        if constexpr (KVB) {
+#pragma unroll
+            for (int j = 0; j < 2 * SS; ++j)
+                Kc[0][ks_row >> 4][ks_c0 + 8 * j][ks_row & 15] = __builtin_bit_cast(uint4, kbs[j]);
+#pragma unroll
+            for (int e = 0; e < SS; ++e) {
+                const int d = vs_d + e * (kHD / SS);
+                uint4 lo, hi;  // dims d and d + 1 of the eight keys
+                uint32_t* pl = &lo.x;
+                uint32_t* ph = &hi.x;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t x = vbs[8 * e + 2 * j], y = vbs[8 * e + 2 * j + 1];
+                    pl[j] = (x & 0xffffu) | (y << 16);
+                    ph[j] = (x >> 16) | (y & 0xffff0000u);
+                }
+                Vc[0][d >> 4][vs_g][(d & 15) ^ (4 * vs_g)] = lo;
+                Vc[0][d >> 4][vs_g][((d + 1) & 15) ^ (4 * vs_g)] = hi;
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const float4 u = kst[2 * i], w = kst[2 * i + 1];
             const float x[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
-            uint4 c[NP];
-            parts8(x, c);
+            uint4 c[3];
+            split3_8(x, c);
 #pragma unroll
             for (int p = 0; p < NP; ++p) Kc[p][ks_row >> 4][ks_c0 + 8 * i][ks_row & 15] = c[p];
         }
@@ -947,17 +988,17 @@ __global__ __launch_bounds__(kFW * 64, 1) void flash_attn_kernel(AttnPrefillArgs
             float x[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[j] = e ? vst[j].y : vst[j].x;
-            uint4 c[NP];
-            parts8(x, c);
+            uint4 c[3];
+            split3_8(x, c);
             const int d = vs_d + e;
 #pragma unroll
             for (int p = 0; p < NP; ++p) Vc[p][d >> 4][vs_g][(d & 15) ^ (4 * vs_g)] = c[p];
         }
     };
-    load_tile(0);
+    load_tile(kv_lo);
     store_tile();
     lds_barrier();
-    for (int kv0 = 0; kv0 < kv_end; kv0 += kKT) {
+    for (int kv0 = kv_lo; kv0 < kv_hi; kv0 += kKT) {
         load_tile(kv0 + kKT);  // in flight during this tile's products
         if (kv0 <= wlast) {    // uniform per wave
             // S^T[key 16 hf + 4 g4 + v][query r16]: the hi.hi products and the smaller part
@@ -1063,20 +1104,29 @@ __global__ __launch_bounds__(kFW * 64, 1) void flash_attn_kernel(AttnPrefillArgs
             }
         }
         lds_barrier();  // every wave is done with this tile
-        if (kv0 + kKT < kv_end) {
+        if (kv0 + kKT < kv_hi) {
             store_tile();
             lds_barrier();
         }
+    }
+    if (!whole) {  // uniform: the piece's output and (max, sum) as they stand, lane by lane
+        const int64_t slot = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+        floatx4* po = reinterpret_cast<floatx4*>(a.part) + (slot * kFW + wave) * 16 * 64 + lane;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) po[64 * t] = o[t];
+        if (g4 == 0) a.part_ml[slot * kQT + wave * 16 + r16] = make_float2(m_run, l_run);
+        return;
     }
     float lr[4];
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) lr[rr] = __shfl(l_run, 4 * g4 + rr);
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) {
-        const int t = t0 + wave * 16 + 4 * g4 + rr;
-        const int tc = min(t, a.T - 1);  // rows past the block compute but store nothing
+        const int row = row0 + wave * 16 + 4 * g4 + rr;
+        const int rc = min(row, rows - 1);  // rows past the block compute but store nothing
+        const int t = rc / grp, h = kh * grp + rc % grp;
         const float inv = 1.0f / lr[rr];
-        const float* gate = a.qkv + static_cast<int64_t>(tc) * a.ld_qkv + static_cast<int64_t>(h) * 2 * kHD + kHD;
+        const float* gate = a.qkv + static_cast<int64_t>(t) * a.ld_qkv + static_cast<int64_t>(h) * 2 * kHD + kHD;
         float* out = a.out + static_cast<int64_t>(t) * (a.NQ * kHD) + static_cast<int64_t>(h) * kHD;
         float mx = 0.0f;
 #pragma unroll
@@ -1084,7 +1134,7 @@ __global__ __launch_bounds__(kFW * 64, 1) void flash_attn_kernel(AttnPrefillArgs
             const int dd = 16 * tt + r16;
             const float y = (o[tt][rr] * inv) * sigmoid_f(gate[dd]);
             mx = fmaxf(mx, fabsf(y));
-            if (t < a.T) {
+            if (row < rows) {
                 if (a.out_tiled) a.out[xt_off(t, h * kHD + dd, a.NQ * kHD)] = y;
                 else out[dd] = y;
             }
@@ -1094,7 +1144,81 @@ __global__ __launch_bounds__(kFW * 64, 1) void flash_attn_kernel(AttnPrefillArgs
             mx = fmaxf(mx, __shfl_xor(mx, 2));
             mx = fmaxf(mx, __shfl_xor(mx, 4));
             mx = fmaxf(mx, __shfl_xor(mx, 8));
-            if (r16 == 0 && t < a.T) a.omax[static_cast<int64_t>(t) * a.NQ + h] = mx;
+            if (r16 == 0 && row < rows) a.omax[static_cast<int64_t>(t) * a.NQ + h] = mx;
+        }
+    }
+}
+
+// Merges the pieces of one 16-row group of a block (grid: wave groups, blocks of all kv
+// heads): every piece's output scaled by e^(its row maximum - the row's), over the sum of the
+// row sums scaled alike, then the gate. The scales of all pieces are formed first, in LDS, so
+// that the partial outputs stream with nothing between their loads; each of the 16 waves takes
+// one output register (dims 16 w + r16 of rows 4 g4 + v, as the flash kernel left them) of
+// every piece, in order.
+template <int W>
+__global__ __launch_bounds__(1024) void flash_combine_kernel(AttnPrefillArgs a, int pieces) {
+    constexpr int QT = 16 * W;
+    const int grp = a.NQ / a.NKV, rows = a.T * grp, nblk = (rows + QT - 1) / QT;
+    const int qt = nblk - 1 - static_cast<int>(blockIdx.y) / a.NKV, kh = blockIdx.y % a.NKV;
+    const int group = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r16 = lane & 15, g4 = lane >> 4;
+    const int row0 = qt * QT + 16 * group;
+    const int kv_end = a.pos0 + min(rows - 1, qt * QT + QT - 1) / grp + 1;
+    const int n = (kv_end + a.piece * kKT - 1) / (a.piece * kKT);
+    if (n <= 1 || row0 >= rows) return;  // uniform: already final, or no rows
+    __shared__ __align__(16) float f_s[kFlashPieces][16];
+    __shared__ float red[64][17], mred[16][16];
+    const int64_t slot0 = static_cast<int64_t>(blockIdx.y) * pieces;
+    // thread (row tid % 16, pieces tid / 16 and 64 + tid / 16): the row's maximum, its scales
+    static_assert(kFlashPieces <= 128, "two pieces per thread");
+    const float2* ml = a.part_ml + slot0 * QT + group * 16 + (tid & 15);
+    const float2 none = make_float2(-INFINITY, 0.0f);
+    const int q0 = tid >> 4;
+    const float2 x0 = q0 < n ? ml[q0 * QT] : none, x1 = 64 + q0 < n ? ml[(64 + q0) * QT] : none;
+    red[q0][tid & 15] = fmaxf(x0.x, x1.x);
+    lds_barrier();
+    float m = -INFINITY;
+    for (int i = 0; i < min(n, 64); ++i) m = fmaxf(m, red[i][tid & 15]);
+    const float f0 = __builtin_amdgcn_exp2f((x0.x - m) * kLog2e);  // 0 for a piece without keys of the row
+    const float f1 = __builtin_amdgcn_exp2f((x1.x - m) * kLog2e);
+    f_s[q0][tid & 15] = f0;
+    f_s[64 + q0][tid & 15] = f1;
+    lds_barrier();
+    red[q0][tid & 15] = x0.y * f0 + x1.y * f1;
+    lds_barrier();
+    floatx4 o = floatx4{0.f, 0.f, 0.f, 0.f};
+    const floatx4* po = reinterpret_cast<const floatx4*>(a.part) + ((slot0 * W + group) * 16 + wave) * 64 + lane;
+#pragma unroll 8
+    for (int q = 0; q < n; ++q)
+        o += po[static_cast<int64_t>(q) * W * 16 * 64] * *reinterpret_cast<const floatx4*>(&f_s[q][4 * g4]);
+    const int dd = 16 * wave + r16;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        float l = 0.0f;
+        for (int i = 0; i < min(n, 64); ++i) l += red[i][4 * g4 + v];
+        const int row = row0 + 4 * g4 + v;
+        const int rc = min(row, rows - 1), t = rc / grp, h = kh * grp + rc % grp;
+        const float gate = a.qkv[static_cast<int64_t>(t) * a.ld_qkv + static_cast<int64_t>(h) * 2 * kHD + kHD + dd];
+        const float y = (o[v] * (1.0f / l)) * sigmoid_f(gate);
+        if (row < rows) {
+            if (a.out_tiled) a.out[xt_off(t, h * kHD + dd, a.NQ * kHD)] = y;
+            else a.out[static_cast<int64_t>(t) * (a.NQ * kHD) + static_cast<int64_t>(h) * kHD + dd] = y;
+        }
+        float mx = fabsf(y);
+        mx = fmaxf(mx, __shfl_xor(mx, 1));
+        mx = fmaxf(mx, __shfl_xor(mx, 2));
+        mx = fmaxf(mx, __shfl_xor(mx, 4));
+        mx = fmaxf(mx, __shfl_xor(mx, 8));
+        if (r16 == 0) mred[wave][4 * g4 + v] = mx;
+    }
+    if (a.omax) {  // uniform: each row's maximum over this head's 256 dims
+        lds_barrier();
+        const int row = row0 + tid;
+        if (tid < 16 && row < rows) {
+            float mx = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mx = fmaxf(mx, mred[i][tid]);
+            a.omax[static_cast<int64_t>(row / grp) * a.NQ + kh * grp + row % grp] = mx;
         }
     }
 }
@@ -1156,19 +1280,79 @@ int64_t attn_prefill_image_floats(int NKV, int pos0, int T) {
     return static_cast<int64_t>(NKV) * attn_prefill_image_tiles(pos0, T) * kImgTile * 4;
 }
 
+int64_t attn_prefill_part_floats(int slots) { return static_cast<int64_t>(slots) * 16 * (kHD + 2); }
+
+// Cuts blocks into pieces where the longest block would outlast an even share of the work.
+// All times in tiles of 32 keys (5.9 us a tile of an fp32 cache, 3.1 us of a bf16 one). One
+// workgroup runs per compute unit and they start longest first, so unsplit blocks take the
+// longest of them or, with more blocks than compute units, the longest pair that shares one.
+// Pieces of c tiles that all start at once take c and about one more for the query rows and
+// the stores; more of them take an even share and about half a piece of unevenness. The merge
+// and its launch are about four more, and a hundredth per piece for its 128 KB of partial
+// output. Split when that is a tenth less. Blocks of up to 64 tiles (2048 keys) stay whole:
+// their output keeps the same bits whatever workspace the caller gives.
+FlashPlan flash_plan(int T, int NQ, int NKV, int pos0, bool kv_bf16) {
+    const FlashPlan whole{0, 0, 0};
+    const int waves = flash_waves(kv_bf16), kQT = 16 * waves;
+    const int grp = NQ / NKV, rows = T * grp, nblk = (rows + kQT - 1) / kQT;
+    const int64_t items = static_cast<int64_t>(nblk) * NKV;
+    const int cu = device_cu_count() * (8 / waves);  // workgroups that run at once
+    // tiles of block b; rank r (longest first) is block nblk - 1 - r / NKV
+    const auto tiles = [&](int64_t b) {
+        return static_cast<int>((pos0 + std::min<int64_t>(rows - 1, b * kQT + kQT - 1) / grp) / kKT + 1);
+    };
+    const int most = tiles(nblk - 1);
+    if (most <= 64 || items >= 2 * cu) return whole;
+    const auto ranked = [&](int64_t r) { return r < items ? tiles(nblk - 1 - r / NKV) : 0; };
+    double best = most;
+    for (int i = 0; i < cu && cu + i < items; ++i) best = std::max<double>(best, ranked(cu - 1 - i) + ranked(cu + i));
+    best *= 0.9;
+    FlashPlan p = whole;
+    for (int pieces = 2; pieces <= kFlashPieces && pieces * items * waves <= kFlashSlots; ++pieces) {
+        const int c = (most + pieces - 1) / pieces;
+        int64_t n = 0, all = 0;
+        for (int b = 0; b < nblk; ++b) {
+            n += static_cast<int64_t>((tiles(b) + c - 1) / c) * NKV;
+            all += static_cast<int64_t>(tiles(b)) * NKV;
+        }
+        const double t = (n <= cu ? c + 1.0 : static_cast<double>(all + n) / cu + 0.6 * c) + 4.0 + 0.01 * n;
+        if (t < best) {
+            best = t;
+            p = FlashPlan{c, (most + c - 1) / c, static_cast<int>((most + c - 1) / c * items * waves)};
+        }
+    }
+    return p;
+}
+
 hipError_t launch_attn_prefill(const AttnPrefillArgs& in, hipStream_t s) {
     AttnPrefillArgs a = in;
     if (a.ROT % 8 == 0) klaunch(attn_prefill_prep_kernel, a.T, 256, 0, s, a);
     else klaunch(attn_prefill_prep_any_kernel, dim3(a.T, a.NQ + a.NKV), 256, 0, s, a);
-    const dim3 grid((a.T + kQT - 1) / kQT, a.NQ);
-    if (a.kv_bf16) {
-        klaunch(flash_attn_kernel<true, false>, grid, kFW * 64, 0, s, a);
-    } else if (a.kv_img) {
+    const int waves = flash_waves(a.kv_bf16), kQT = 16 * waves;
+    const int blocks = (a.T * (a.NQ / a.NKV) + kQT - 1) / kQT * a.NKV;
+    FlashPlan p{0, 0, 0};
+    if (a.part) p = flash_plan(a.T, a.NQ, a.NKV, a.pos0, a.kv_bf16);
+    if (p.slots > a.part_slots) p = FlashPlan{0, 0, 0};
+    a.piece = p.piece;
+    a.part_ml = p.pieces ? reinterpret_cast<float2*>(a.part + static_cast<int64_t>(p.slots) * 16 * kHD) : nullptr;
+    const dim3 grid = p.pieces ? dim3(p.pieces, blocks) : dim3(blocks);
+    const bool img = !a.kv_bf16 && a.kv_img;
+    if (img) {
         a.img_tiles = attn_prefill_image_tiles(a.pos0, a.T);
         klaunch(attn_kv_image_kernel, dim3(a.img_tiles, a.NKV), 256, 0, s, a);
-        klaunch(flash_attn_kernel<false, true>, grid, kFW * 64, 0, s, a);
+    }
+    if (p.pieces) {
+        if (a.kv_bf16) klaunch(flash_attn_kernel<true, false, true>, grid, 64 * waves, 0, s, a);
+        else if (img) klaunch(flash_attn_kernel<false, true, true>, grid, 64 * waves, 0, s, a);
+        else klaunch(flash_attn_kernel<false, false, true>, grid, 64 * waves, 0, s, a);
+        if (a.kv_bf16) klaunch(flash_combine_kernel<flash_waves(true)>, dim3(waves, blocks), 1024, 0, s, a, p.pieces);
+        else klaunch(flash_combine_kernel<flash_waves(false)>, dim3(waves, blocks), 1024, 0, s, a, p.pieces);
+    } else if (a.kv_bf16) {
+        klaunch(flash_attn_kernel<true, false, false>, grid, 64 * waves, 0, s, a);
+    } else if (img) {
+        klaunch(flash_attn_kernel<false, true, false>, grid, 64 * waves, 0, s, a);
     } else {
-        klaunch(flash_attn_kernel<false, false>, grid, kFW * 64, 0, s, a);
+        klaunch(flash_attn_kernel<false, false, false>, grid, 64 * waves, 0, s, a);
     }
     return hipGetLastError();
 }

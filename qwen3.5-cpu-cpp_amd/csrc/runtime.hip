@@ -761,8 +761,11 @@ PrefillPlan plan_prefill(const q35_dims& d, int tb, int64_t logits_width, bool e
     p.proj = take(T * proj_width(d));
     p.mix = take(TP * std::max(VD, QD));
     p.hb = take(TP * I);
+    // (the attention's share has room for half of the largest split of its key ranges, 66 MB:
+    // what a few tokens on a long context need; at 4096 tokens the GDN share is the larger one)
     p.ws_n = std::max(q35k::gdn_prefill_workspace_floats(d.gdn_k_heads, d.gdn_v_heads, tb),
-                      q35k::attn_prefill_workspace_floats(d.attn_q_heads, tb));
+                      q35k::attn_prefill_workspace_floats(d.attn_q_heads, tb) +
+                          q35k::attn_prefill_part_floats(q35k::kFlashSlots / 2));
     p.ws = take(p.ws_n);
     p.logits = take(static_cast<int64_t>(p.lr) * logits_width);
     p.ids = take(T);
@@ -1198,10 +1201,17 @@ q35_status prefill_block(q35_model* m, const PrefillPlan& p, int pos0, int T, in
             a.kv_bf16 = m->kv_elem == 2;
             a.rope_cs = m->rope_cs;
             a.Qa = ws;
-            // the pre-split key / value tiles where they fit in the rest of the workspace
-            // (the GDN layers' share is the larger one at 2B shapes: up to ~35k keys)
-            const int64_t qa_n = q35k::attn_prefill_workspace_floats(NQ, T);
-            if (!a.kv_bf16 && qa_n + q35k::attn_prefill_image_floats(NKV, pos0, T) <= p.ws_n) a.kv_img = ws + qa_n;
+            // the partial outputs of split key ranges (few tokens over many keys), then the
+            // pre-split key / value tiles where they fit in the rest of the workspace (the GDN
+            // layers' share is the larger one at 2B shapes: up to ~35k keys)
+            int64_t used = q35k::attn_prefill_workspace_floats(NQ, T);
+            const int slots = q35k::flash_plan(T, NQ, NKV, pos0, a.kv_bf16).slots;
+            if (slots && used + q35k::attn_prefill_part_floats(slots) <= p.ws_n) {
+                a.part = ws + used;
+                a.part_slots = slots;
+                used += q35k::attn_prefill_part_floats(slots);
+            }
+            if (!a.kv_bf16 && used + q35k::attn_prefill_image_floats(NKV, pos0, T) <= p.ws_n) a.kv_img = ws + used;
             a.out = mix;
             a.omax = mix_max;
             a.out_tiled = p.tiled;
