@@ -838,7 +838,7 @@ __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma_bf16_kernel(const int* 
     }
 }
 
-// ---- fp32 caches, GQA 8: both products on v_mfma_f32_4x4x1_16b_f32 ----------------------
+// ---- fp32 caches, GQA 4 and 8, and bf16 caches, GQA 4: both products on v_mfma_f32_4x4x1_16b_f32 ----------------------
 // 16x16x4 products would use 8 of their 16 columns (8 query heads); the 4x4x1 instruction
 // holds 16 independent 4 x 4 blocks, so every lane carries a useful product. Lane l = 16 g + 4 pg + j (block b = l / 4 = pg + 4 g, A row / B column j):
 //   S = K.Q^T: A = K[row 4 pg + j][dim], B = Q[head 4 hg + j][dim] for the dims 16 u + 4 g + e
@@ -853,6 +853,11 @@ __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma_bf16_kernel(const int* 
 //   LDS per wave.
 // 256 products of 4x4x1 per 16-position tile against 128 of 16x16x4: measured about 10-11
 // cycles against 32 per instruction, so each tile's products take ~2.5k cycles instead of ~4k.
+// A bf16 cache's rows are widened (exactly) as they are used: K 16 bytes a lane, dims 32 c +
+// 8 g .. + 7 of row 4 pg + j in register c; V rows as whole 512-byte rows. (Its products for
+// groups of 4 on the 16-bit cores, as attn_mfma_bf16_kernel has them, are as fast but
+// further from float64, 2.8e-7 against 2.25e-7 at 3k positions: those cores cut the low bits
+// of what they add up, always downwards.)
 __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
 }
@@ -873,24 +878,25 @@ __device__ __forceinline__ float pg_sum(float v) {
     return v + dpp_f<0x128>(v);
 }
 
-template <bool ML>
+template <int GRP, bool ML, bool KVB>
 __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma4_kernel(const int* pos_dev, int pos_val, const float* qg,
                                                             const float* k_new, const float* v_new,
                                                             const float* q_norm, const float* k_norm,
                                                             AttnDecodeArgs a) {
     set_lead(a, pos_dev, pos_val, qg, k_new, v_new, q_norm, k_norm);
     if (ML) attn_select_layer(a, blockIdx.z);
-    constexpr int GRP = 8, TP = 16;
+    constexpr int TP = 16, HG = (GRP + 3) / 4;  // groups of 4 query heads
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar loop bounds
     const int n16 = lane & 15, g = lane >> 4, jj = lane & 3, pg = (lane >> 2) & 3;
     const int split = blockIdx.x, kh = blockIdx.y;
-    // the query-side rows first (rows of this wave: q heads wave, wave + 4, and row 8 the
-    // appended key); they do not depend on the position
-    float4 px[3], pw[3];
+    // the query-side rows first (rows of this wave: q heads wave, wave + 4, .., and row
+    // GRP the appended key); they do not depend on the position
+    constexpr int NI = GRP / kMW + 1;
+    float4 px[NI], pw[NI];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const int r = min(wave + i * kMW, GRP);  // row 8 = the new key
+    for (int i = 0; i < NI; ++i) {
+        const int r = min(wave + i * kMW, GRP);  // row GRP = the new key
         const float* src = r < GRP ? a.qg + static_cast<int64_t>(kh * GRP + r) * 2 * kHD
                                    : a.k_new + static_cast<int64_t>(kh) * kHD;
         px[i] = *reinterpret_cast<const float4*>(src + lane * 4);
@@ -920,18 +926,20 @@ __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma4_kernel(const int* pos_
     const bool has_new = owns_new && w0 < w1 && w1 == n;  // empty waves also end at n
     const int wl = has_new ? w1 - 1 : w1;
 
-    const float* Kc = kcache + hoff;
-    const float* Vc = vcache + hoff;
+    const float* Kc = kcache + (KVB ? 0 : hoff);
+    const float* Vc = vcache + (KVB ? 0 : hoff);
+    const uint16_t* Kb = reinterpret_cast<const uint16_t*>(kcache) + hoff;
+    const uint16_t* Vb = reinterpret_cast<const uint16_t*>(vcache) + hoff;
     const float sc = 1.0f / sqrtf(static_cast<float>(kHD));
 
-    __shared__ float4 qs[2][16][4][4];       // Q operand: [hg][u][j][g] = Q[4 hg + j][16 u + 4 g .. + 3]
+    __shared__ float4 qs[HG][16][4][4];      // Q operand: [hg][u][j][g] = Q[4 hg + j][16 u + 4 g .. + 3]
     __shared__ float4 ks[kHD / 4], vs[kHD / 4];  // the appended rows
-    __shared__ float4 pl[kMW][2][4][4];      // softmax weights of a tile: [hg][j][t] = P[4 hg + j][4 t .. + 3]
+    __shared__ float4 pl[kMW][HG][4][4];      // softmax weights of a tile: [hg][j][t] = P[4 hg + j][4 t .. + 3]
     __shared__ float os[kMW][GRP][kHD];
     __shared__ float ml_s[kMW][GRP][2];
 
-    // ---- prologue (the rows requested above: q heads wave, wave + 4 of this wave, the key
-    // on wave 0 and the value on wave 1 of the workgroup holding pos): the RoPE table row,
+    // ---- prologue (the rows requested above: q heads wave, wave + 4, .. of this wave, the key
+    // on wave GRP % 4 and the value on wave 1 of the workgroup holding pos): the RoPE table row,
     // then the first K / V tiles
     const int ci = (lane * 4) % max(half, 4);  // table column of this lane's first dim
     float4 cs4 = make_float4(1.f, 1.f, 1.f, 1.f), sn4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -944,20 +952,31 @@ __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma4_kernel(const int* pos_
     // register p. Loads are issued unconditionally (a load under a branch makes the
     // wait-count pass wait for all outstanding loads at the join); past the end of the range
     // every lane reads the same 16 bytes of a valid row.
-    float4 kA[16], vr[16];
+    // (bf16: K row n16, dims 32 c + 8 g .. + 7 in register c; V rows the same)
+    typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+    constexpr int NK = KVB ? 8 : 16;
+    using KReg = typename std::conditional<KVB, u4, float4>::type;
+    using VReg = typename std::conditional<KVB, u2, float4>::type;
+    KReg kA[NK];
+    VReg vr[16];
     const int last = max(wl - 1, 0);  // a valid row to clamp to
-    auto loadK = [&](float4 (&kr)[16], int p0) {
+    auto loadK = [&](KReg (&kr)[NK], int p0) {
         const int mask = -static_cast<int>(p0 < wl);  // all ones while live (no branch)
         const int64_t row = min(p0 + n16, last);
 #pragma unroll
-        for (int u = 0; u < 16; ++u) kr[u] = load_stream(Kc + row * kHD + ((16 * u + 4 * g) & mask));
+        for (int u = 0; u < NK; ++u) {
+            if constexpr (KVB) kr[u] = __builtin_nontemporal_load(reinterpret_cast<const u4*>(Kb + row * kHD + ((32 * u + 8 * g) & mask)));
+            else kr[u] = load_stream(Kc + row * kHD + ((16 * u + 4 * g) & mask));
+        }
     };
     auto loadV = [&](int p0) {
         const int mask = -static_cast<int>(p0 < wl);
 #pragma unroll
         for (int p = 0; p < TP; ++p) {
             const int64_t row = min((p0 + p) & mask, last) | (last & ~mask);
-            vr[p] = load_stream(Vc + row * kHD + ((4 * lane) & mask));
+            if constexpr (KVB) vr[p] = __builtin_nontemporal_load(reinterpret_cast<const u2*>(Vb + row * kHD + ((4 * lane) & mask)));
+            else vr[p] = load_stream(Vc + row * kHD + ((4 * lane) & mask));
         }
     };
     loadK(kA, w0);
@@ -965,36 +984,50 @@ __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma4_kernel(const int* pos_
 
     // ---- Q operand and the appended rows
     if (!a.rope_cs) rope_cs4(a.theta, ROT, pos, lane, cs4, sn4);  // double-precision angles
+    // stores the lane's 4 dims of the appended row and returns them as the cache holds them
+    auto append = [&](float* cache, float4 y) {
+        const int64_t off = hoff + static_cast<int64_t>(pos) * kHD + lane * 4;
+        if constexpr (KVB) {
+            const uint32_t b0 = f32_to_bf16(y.x), b1 = f32_to_bf16(y.y), b2 = f32_to_bf16(y.z), b3 = f32_to_bf16(y.w);
+            const uint2 w = make_uint2(b0 | (b1 << 16), b2 | (b3 << 16));
+            *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(cache) + off) = w;
+            return make_float4(bf16_lo(w.x), bf16_hi(w.x), bf16_lo(w.y), bf16_hi(w.y));
+        } else {
+            *reinterpret_cast<float4*>(cache + off) = y;
+            return y;
+        }
+    };
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
+    for (int i = 0; i < NI; ++i) {
         const int r = wave + i * kMW;
         if (r > GRP || (r == GRP && !owns_new)) continue;  // uniform per wave
-        const float4 y = norm_rope_row(px[i], pw[i], cs4, sn4, lane, ROT, a.eps);
+        float4 y = norm_rope_row(px[i], pw[i], cs4, sn4, lane, ROT, a.eps);
         if (r < GRP) {
             qs[r >> 2][lane >> 2][r & 3][lane & 3] = y;  // dims 4 lane .. + 3 of head r
         } else {
-            *reinterpret_cast<float4*>(a.k_cache + hoff + static_cast<int64_t>(pos) * kHD + lane * 4) = y;
-            ks[lane] = y;
+            ks[lane] = append(a.k_cache, y);
         }
     }
-    if (owns_new && wave == 1) {
-        *reinterpret_cast<float4*>(a.v_cache + hoff + static_cast<int64_t>(pos) * kHD + lane * 4) = vn4;
-        vs[lane] = vn4;
-    }
+    if (owns_new && wave == 1) vs[lane] = append(a.v_cache, vn4);
     // LDS-only barrier: the K / V tiles in flight are not waited for here
     lds_barrier();
 
-    floatx4 O[2][4];  // [hg][c]: register i = O[4 hg + i][4 lane + c]
+    floatx4 O[HG][4];  // [hg][c]: register i = O[4 hg + i][4 lane + c]
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < HG; ++h)
 #pragma unroll
         for (int c = 0; c < 4; ++c) O[h][c] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.0f, 0.0f};  // of heads jj + 4 hg
+    float m_run[HG], l_run[HG];  // of heads jj + 4 hg
+#pragma unroll
+    for (int h = 0; h < HG; ++h) {
+        m_run[h] = -INFINITY;
+        l_run[h] = 0.0f;
+    }
 
     // rescale the accumulators of heads 4 hg + i by the factors f of lanes i (heads i + 4 hg)
-    auto rescale = [&](const float (&f)[2]) {
+    auto rescale = [&](const float (&f)[HG]) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < HG; ++h) {
             float fh[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) fh[i] = __shfl(f[h], i);
@@ -1005,31 +1038,39 @@ __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma4_kernel(const int* pos_
         }
     };
 
-    auto tile = [&](float4 (&kr)[16], int p0, auto more) {
-        floatx4 Sx[2][4];  // [hg][e]: eight independent accumulation chains
+    auto tile = [&](KReg (&kr)[NK], int p0, auto more) {
+        floatx4 Sx[HG][4];  // [hg][e]: independent accumulation chains
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < HG; ++h)
 #pragma unroll
             for (int e = 0; e < 4; ++e) Sx[h][e] = floatx4{0.f, 0.f, 0.f, 0.f};
+        auto dims4 = [&](float4 k, int u, int q4) {  // k: dims 16 u + 4 q4 .. + 3 of the lane's row
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const float4 k = kr[u];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const float4 q = qs[h][u][jj][g];
+            for (int h = 0; h < HG; ++h) {
+                const float4 q = qs[h][u][jj][q4];
                 Sx[h][0] = mfma4(k.x, q.x, Sx[h][0]);
                 Sx[h][1] = mfma4(k.y, q.y, Sx[h][1]);
                 Sx[h][2] = mfma4(k.z, q.z, Sx[h][2]);
                 Sx[h][3] = mfma4(k.w, q.w, Sx[h][3]);
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < NK; ++u) {
+            if constexpr (KVB) {  // dims 32 u + 8 g .. + 7
+                const u4 k = kr[u];
+                dims4(make_float4(bf16_lo(k.x), bf16_hi(k.x), bf16_lo(k.y), bf16_hi(k.y)), 2 * u + (g >> 1), 2 * (g & 1));
+                dims4(make_float4(bf16_lo(k.z), bf16_hi(k.z), bf16_lo(k.w), bf16_hi(k.w)), 2 * u + (g >> 1), 2 * (g & 1) + 1);
+            } else {
+                dims4(kr[u], u, g);
             }
             // keep the Q operand reads close to their use (a few in flight, not all 32)
             if ((u & 3) == 3) __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (decltype(more)::value) loadK(kr, p0 + TP);
         // s[h][i]: position p0 + 4 pg + i, head 4 h + jj (the dim quarters summed)
-        float s[2][4], tm[2];
+        float s[HG][4], tm[HG];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < HG; ++h) {
             const floatx4 S = (Sx[h][0] + Sx[h][1]) + (Sx[h][2] + Sx[h][3]);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -1040,9 +1081,9 @@ __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma4_kernel(const int* pos_
         }
         // the reference max moves only when a score exceeds it by more than 8 (the weights
         // exp(s - m) stay below e^8, far from overflow), so the accumulators are rarely rescaled
-        float f[2], p[2][4];
+        float f[HG], p[HG][4];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < HG; ++h) {
             const float m_new = tm[h] > m_run[h] + 8.0f ? tm[h] : m_run[h];
             f[h] = expf(m_run[h] - m_new);
             float ps = 0.0f;
@@ -1054,53 +1095,70 @@ __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma4_kernel(const int* pos_
             l_run[h] = l_run[h] * f[h] + pg_sum(ps);
             m_run[h] = m_new;
         }
-        if (__any(f[0] != 1.0f || f[1] != 1.0f)) rescale(f);
+        if (__any(f[0] != 1.0f || f[HG - 1] != 1.0f)) rescale(f);
         // P to the A operand layout: the lanes of dim quarter 0 store their 4 positions of
         // heads jj, jj + 4; every lane reads the 16 positions of its heads (same wave: LDS
         // operations complete in order)
         if (g == 0) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) pl[wave][h][jj][pg] = make_float4(p[h][0], p[h][1], p[h][2], p[h][3]);
+            for (int h = 0; h < HG; ++h) pl[wave][h][jj][pg] = make_float4(p[h][0], p[h][1], p[h][2], p[h][3]);
         }
         __builtin_amdgcn_wave_barrier();
-        float4 pv[2][4];
+        float4 pv[HG][4];
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < HG; ++h)
 #pragma unroll
             for (int t = 0; t < 4; ++t) pv[h][t] = pl[wave][h][jj][t];
+        // GRP 4: the tile's products from zero, then one addition to the total (fewer roundings
+        // at the total's size)
+        floatx4 D[HG][4];
+#pragma unroll
+        for (int h = 0; h < HG; ++h)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) D[h][c] = GRP == 4 ? floatx4{0.f, 0.f, 0.f, 0.f} : O[h][c];
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float4 v = vr[4 * t + e];
+                float4 v;
+                if constexpr (KVB) {
+                    const u2 w = vr[4 * t + e];
+                    v = make_float4(bf16_lo(w.x), bf16_hi(w.x), bf16_lo(w.y), bf16_hi(w.y));
+                } else {
+                    v = vr[4 * t + e];
+                }
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
+                for (int h = 0; h < HG; ++h) {
                     const float pa = e == 0 ? pv[h][t].x : e == 1 ? pv[h][t].y : e == 2 ? pv[h][t].z : pv[h][t].w;
-                    O[h][0] = mfma4(pa, v.x, O[h][0]);
-                    O[h][1] = mfma4(pa, v.y, O[h][1]);
-                    O[h][2] = mfma4(pa, v.z, O[h][2]);
-                    O[h][3] = mfma4(pa, v.w, O[h][3]);
+                    D[h][0] = mfma4(pa, v.x, D[h][0]);
+                    D[h][1] = mfma4(pa, v.y, D[h][1]);
+                    D[h][2] = mfma4(pa, v.z, D[h][2]);
+                    D[h][3] = mfma4(pa, v.w, D[h][3]);
                 }
             }
+#pragma unroll
+        for (int h = 0; h < HG; ++h)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) O[h][c] = GRP == 4 ? O[h][c] + D[h][c] : D[h][c];
         if constexpr (decltype(more)::value) loadV(p0 + TP);
     };
     int p0 = w0;
     for (; p0 + TP < wl; p0 += TP) tile(kA, p0, std::true_type{});
     if (p0 < wl) tile(kA, p0, std::false_type{});  // the last tile requests nothing more
 
-    if (has_new) {  // position pos: each lane's 4 dims for the 8 heads, then a halving butterfly
+    if (has_new) {  // position pos: each lane's 4 dims for the query heads, then a halving butterfly
         const float4 kn = ks[lane];
-        fvec<8> d;
+        fvec<GRP> d;
 #pragma unroll
         for (int h = 0; h < GRP; ++h) {
             const float4 q = qs[h >> 2][lane >> 2][h & 3][lane & 3];
             d[h] = ((q.x * kn.x + q.y * kn.y) + q.z * kn.z) + q.w * kn.w;
         }
-        const float dh = butterfly<8, 32>(d, lane);  // head lane / 8 on every lane
-        float f[2], pn[2];
+        const float dh = butterfly<GRP, 32>(d, lane);  // head lane / (64 / GRP) on every lane
+        float f[HG], pn[HG];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const float sn = __shfl(dh, 8 * (jj + 4 * h)) * sc;
+        for (int h = 0; h < HG; ++h) {
+            const float sn = __shfl(dh, 64 / GRP * (jj + 4 * h)) * sc;
             const float m_new = sn > m_run[h] + 8.0f ? sn : m_run[h];
             f[h] = expf(m_run[h] - m_new);
             pn[h] = expf(sn - m_new);
@@ -1110,7 +1168,7 @@ __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma4_kernel(const int* pos_
         rescale(f);
         const float4 v = vs[lane];
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < HG; ++h)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float ph = __shfl(pn[h], i);
@@ -1125,14 +1183,14 @@ __global__ __launch_bounds__(kMW * 64, 2) void attn_mfma4_kernel(const int* pos_
     // workgroup maximum and the four are summed in a fixed order
     if (lane < 4) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < HG; ++h) {
             ml_s[wave][lane + 4 * h][0] = m_run[h];
             ml_s[wave][lane + 4 * h][1] = l_run[h];
         }
     }
     lds_barrier();
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < HG; ++h)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int hd = 4 * h + i;
@@ -1253,15 +1311,30 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const int* pos_dev, c
 
 template <int GRP>
 hipError_t launch_partial_grp(const AttnDecodeArgs& a, hipStream_t s) {
-    if (GRP == 8 && a.ROT % 32 == 0 && a.ROT > 0 && !attn_force_valu()) {
-        dim3 grid(a.n_splits, a.NKV, a.n_layers > 0 ? a.n_layers : 1);
-        auto go = [&](auto k) {
-            klaunch(k, grid, kMW * 64, 0, s, a.pos_dev, a.pos_val, a.qg, a.k_new, a.v_new, a.q_norm, a.k_norm, a);
-        };
-        const bool ml = grid.z > 1;
-        if (a.kv_bf16) ml ? go(attn_mfma_bf16_kernel<true>) : go(attn_mfma_bf16_kernel<false>);
-        else ml ? go(attn_mfma4_kernel<true>) : go(attn_mfma4_kernel<false>);
-        return hipGetLastError();
+    // The matrix-core kernels serve groups of 4 and 8 heads. A group of 4 takes them too,
+    // vector ALU against matrix cores, 6 layers x 2 kv heads: bf16 cache 100 positions 12.4 / 11.5
+    // us, 2k 15.6 / 14.1, 3k 26.0 / 18.0, 8k 33.3 / 24.1, 32k 73.9 / 69.5; fp32 12.4 / 11.5, 2k
+    // 18.5 / 16.3, 8k 42.9 / 38.7, 32k 126.7 / 125.7; one layer at 32k 30.2 / 27.8 fp32 and 22.9 /
+    // 20.0 bf16; the same distance from float64 (2.2e-7 to 2.5e-7). bf16 K rows are read 16 bytes
+    // at a time (the vector kernel's 8).
+    if constexpr (GRP == 4 || GRP == 8) {
+        const auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+        const bool wide = GRP == 8 || !a.kv_bf16 || (a16(a.k_cache) && a16(a.v_cache));
+        if (a.ROT % 32 == 0 && a.ROT > 0 && wide && !attn_force_valu()) {
+            dim3 grid(a.n_splits, a.NKV, a.n_layers > 0 ? a.n_layers : 1);
+            auto go = [&](auto k) {
+                klaunch(k, grid, kMW * 64, 0, s, a.pos_dev, a.pos_val, a.qg, a.k_new, a.v_new, a.q_norm, a.k_norm, a);
+            };
+            const bool ml = grid.z > 1;
+            if (!a.kv_bf16) {
+                ml ? go(attn_mfma4_kernel<GRP, true, false>) : go(attn_mfma4_kernel<GRP, false, false>);
+            } else if constexpr (GRP == 8) {
+                ml ? go(attn_mfma_bf16_kernel<true>) : go(attn_mfma_bf16_kernel<false>);
+            } else {
+                ml ? go(attn_mfma4_kernel<GRP, true, true>) : go(attn_mfma4_kernel<GRP, false, true>);
+            }
+            return hipGetLastError();
+        }
     }
     constexpr int LPP = GRP <= 4 ? 16 : 32;
     dim3 grid(a.n_splits, a.NKV, a.n_layers > 0 ? a.n_layers : 1);
