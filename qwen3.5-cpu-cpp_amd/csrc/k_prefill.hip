@@ -597,6 +597,205 @@ __global__ __launch_bounds__(256, 2) void gdn_out_kernel(GdnPrefillArgs a) {
     }
 }
 
+// ------------------------------------------------------------------ GDN over few tokens
+// sum over the 8 lanes l, l ^ 8, ..., l ^ 56 (the row groups of one column quad)
+__device__ __forceinline__ float rowgroup8_sum(float v) {
+    v += dpp_f<0x128>(v);
+    auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), false, false);
+    v = __builtin_bit_cast(float, static_cast<int>(r[0])) + __builtin_bit_cast(float, static_cast<int>(r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), false, false);
+    return __builtin_bit_cast(float, static_cast<int>(r[0])) + __builtin_bit_cast(float, static_cast<int>(r[1]));
+}
+
+constexpr int kShortT = 48;      // most tokens
+constexpr int kShortRun = 4;     // tokens per conv run
+constexpr int kShortThreads = 512;
+
+// grid (VH), 512 threads: a whole block of up to kShortT tokens of one v-head in one launch,
+// token by token like the decode step, the state in registers throughout.
+//   conv   runs of 4 tokens x 4 channels of the head's q, k and v, SiLU, into LDS; beta and
+//          the decay of each token
+//   norm   each half-wave l2-normalises q or k rows in place (q also scaled by DK^-1/2)
+//   scan   waves 0-3 own 32 state columns each: lane l rows 16 (l / 8) .. + 15 of columns
+//          4 (l % 8) .. + 3 (as gdn_wave_kernel); the readout takes v's place in LDS
+//   out    each half-wave one token: the gated rmsnorm (or the raw readout), row maximum
+// The chunked kernels take the time of one chunk of 64 however few tokens there are, most of
+// it serial latency; a 32-token prompt of the 0.8B shape went from 3.59 to 3.11 ms.
+__global__ __launch_bounds__(kShortThreads) void gdn_short_kernel(GdnPrefillArgs a) {
+    const int vh = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int rep = a.VH / a.KH, kh = vh / rep;
+    const int KD = a.KH * kD, CONV = 2 * KD + a.VH * kD;
+    __shared__ __align__(16) float qs[kShortT * kD], ks[kShortT * kD], vs[kShortT * kD];  // vs: v, then the readout
+    __shared__ float al[kShortT], be[kShortT];
+    float* S = a.state + static_cast<int64_t>(vh) * kD * kD;
+
+    // the state slice of the scan waves, requested first
+    constexpr int RR = 16;
+    const int rg = lane >> 3, col0 = 32 * wave + 4 * (lane & 7);
+    float4 s[RR];
+    if (wave < 4) {
+#pragma unroll
+        for (int i = 0; i < RR; ++i) s[i] = *reinterpret_cast<const float4*>(S + (RR * rg + i) * kD + col0);
+    }
+    // ---- conv
+    const int runs = (a.T + kShortRun - 1) / kShortRun;
+    for (int item = tid; item < 96 * runs; item += kShortThreads) {
+        const int run = item / 96, quad = item - 96 * run;  // quads 0-31 q, 32-63 k, 64-95 v
+        const int part = quad >> 5, c4 = 4 * (quad & 31), t0 = kShortRun * run;
+        const int ch = (part == 0 ? kh * kD : part == 1 ? KD + kh * kD : 2 * KD + vh * kD) + c4;
+        float4 x[kShortRun + 3], w[4];
+#pragma unroll
+        for (int j = 0; j < kShortRun + 3; ++j) {
+            const int t = t0 - 3 + j;  // t < 0: the conv ring
+            const float* p = t >= 0 ? a.qkv + static_cast<int64_t>(min(t, a.T - 1)) * a.ld_qkv + ch
+                                    : a.conv_ring + static_cast<int64_t>((a.pos0 + t) & 3) * CONV + ch;
+            x[j] = *reinterpret_cast<const float4*>(p);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = *reinterpret_cast<const float4*>(a.conv_w + static_cast<int64_t>(ch + e) * 4);
+        float* dst = (part == 0 ? qs : part == 1 ? ks : vs) + t0 * kD + c4;
+#pragma unroll
+        for (int j = 0; j < kShortRun; ++j) {
+            float y[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                auto at = [&](const float4& q) { return e == 0 ? q.x : e == 1 ? q.y : e == 2 ? q.z : q.w; };
+                float acc = 0.0f;
+                acc += w[e].x * at(x[j]);
+                acc += w[e].y * at(x[j + 1]);
+                acc += w[e].z * at(x[j + 2]);
+                acc += w[e].w * at(x[j + 3]);
+                y[e] = silu_f(acc);
+            }
+            if (t0 + j < a.T) *reinterpret_cast<float4*>(dst + j * kD) = make_float4(y[0], y[1], y[2], y[3]);
+        }
+    }
+    if (tid < a.T) {
+        const float g = -expf(a.A_log[vh]) * softplus_f(a.a[static_cast<int64_t>(tid) * a.ld_ba + vh] + a.dt_bias[vh]);
+        al[tid] = expf(g);
+        be[tid] = sigmoid_f(a.b[static_cast<int64_t>(tid) * a.ld_ba + vh]);
+    }
+    lds_barrier();
+    // ---- l2norm (eps 1e-6, sums of squares in double)
+    const int half = tid >> 5, l32 = tid & 31;  // 16 half-waves
+    for (int r = half; r < 2 * a.T; r += kShortThreads / 32) {
+        float* row = (r < a.T ? qs + r * kD : ks + (r - a.T) * kD) + 4 * l32;
+        const float4 x = *reinterpret_cast<const float4*>(row);
+        double ss = static_cast<double>(x.x) * x.x + static_cast<double>(x.y) * x.y + static_cast<double>(x.z) * x.z +
+                    static_cast<double>(x.w) * x.w;
+        ss = half_wave_sum(ss);
+        const float inv = 1.0f / sqrtf(static_cast<float>(ss) + 1e-6f);
+        const float qsc = r < a.T ? 1.0f / sqrtf(static_cast<float>(kD)) : 1.0f;
+        *reinterpret_cast<float4*>(row) =
+            make_float4((x.x * inv) * qsc, (x.y * inv) * qsc, (x.z * inv) * qsc, (x.w * inv) * qsc);
+    }
+    // the block's last three raw inputs into the ring (one v-head per k-head: nobody else
+    // reads these channels; else gdn_ring_kernel writes it)
+    if (rep == 1 && tid < 3 * 96) {
+        const int quad = tid % 96, part = quad >> 5, t = a.T - 1 - tid / 96;
+        const int ch = (part == 0 ? kh * kD : part == 1 ? KD + kh * kD : 2 * KD + vh * kD) + 4 * (quad & 31);
+        if (t >= 0)
+            *reinterpret_cast<float4*>(a.conv_ring + static_cast<int64_t>((a.pos0 + t) & 3) * CONV + ch) =
+                *reinterpret_cast<const float4*>(a.qkv + static_cast<int64_t>(t) * a.ld_qkv + ch);
+    }
+    lds_barrier();
+    // ---- scan
+    if (wave < 4) {
+        float4 q4[RR / 4], k4[RR / 4], v4;
+        auto read = [&](int t) {
+#pragma unroll
+            for (int j = 0; j < RR / 4; ++j) {
+                q4[j] = *reinterpret_cast<const float4*>(qs + t * kD + RR * rg + 4 * j);
+                k4[j] = *reinterpret_cast<const float4*>(ks + t * kD + RR * rg + 4 * j);
+            }
+            v4 = *reinterpret_cast<const float4*>(vs + t * kD + col0);
+        };
+        read(0);
+#pragma unroll 1
+        for (int t = 0; t < a.T; ++t) {
+            const float alpha = al[t], beta = be[t];
+            float qn[RR], kn[RR];
+#pragma unroll
+            for (int j = 0; j < RR / 4; ++j) {
+                qn[4 * j] = q4[j].x, qn[4 * j + 1] = q4[j].y, qn[4 * j + 2] = q4[j].z, qn[4 * j + 3] = q4[j].w;
+                kn[4 * j] = k4[j].x, kn[4 * j + 1] = k4[j].y, kn[4 * j + 2] = k4[j].z, kn[4 * j + 3] = k4[j].w;
+            }
+            const float4 v = v4;
+            if (t + 1 < a.T) read(t + 1);  // uniform: the next token's rows while this one's are used
+            float4 km = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int i = 0; i < RR; ++i) {
+                s[i].x *= alpha;
+                s[i].y *= alpha;
+                s[i].z *= alpha;
+                s[i].w *= alpha;
+                km.x += s[i].x * kn[i];
+                km.y += s[i].y * kn[i];
+                km.z += s[i].z * kn[i];
+                km.w += s[i].w * kn[i];
+            }
+            km.x = rowgroup8_sum(km.x);
+            km.y = rowgroup8_sum(km.y);
+            km.z = rowgroup8_sum(km.z);
+            km.w = rowgroup8_sum(km.w);
+            const float4 d = make_float4((v.x - km.x) * beta, (v.y - km.y) * beta, (v.z - km.z) * beta, (v.w - km.w) * beta);
+            float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int i = 0; i < RR; ++i) {
+                s[i].x += kn[i] * d.x;
+                s[i].y += kn[i] * d.y;
+                s[i].z += kn[i] * d.z;
+                s[i].w += kn[i] * d.w;
+                o.x += s[i].x * qn[i];
+                o.y += s[i].y * qn[i];
+                o.z += s[i].z * qn[i];
+                o.w += s[i].w * qn[i];
+            }
+            o.x = rowgroup8_sum(o.x);
+            o.y = rowgroup8_sum(o.y);
+            o.z = rowgroup8_sum(o.z);
+            o.w = rowgroup8_sum(o.w);
+            if (rg == 0) *reinterpret_cast<float4*>(vs + t * kD + col0) = o;
+        }
+#pragma unroll
+        for (int i = 0; i < RR; ++i) *reinterpret_cast<float4*>(S + (RR * rg + i) * kD + col0) = s[i];
+    }
+    lds_barrier();
+    // ---- out: half-wave h takes tokens h, h + 16, ..; lane l columns l, l + 32, l + 64, l + 96
+    for (int t = half; t < a.T; t += kShortThreads / 32) {
+        float o[4], z[4] = {0.f, 0.f, 0.f, 0.f}, nw[4] = {1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            o[e] = vs[t * kD + l32 + 32 * e];
+            if (a.norm_w) {  // uniform
+                z[e] = a.z[static_cast<int64_t>(t) * a.ld_z + vh * kD + l32 + 32 * e];
+                nw[e] = a.norm_w[l32 + 32 * e];
+            }
+        }
+        double ss = 0.0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss += static_cast<double>(o[e]) * o[e];
+        ss = half_wave_sum(ss);
+        const float inv = 1.0f / sqrtf(static_cast<float>(ss / kD) + a.eps);
+        float mx = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int c = vh * kD + l32 + 32 * e;
+            const float y = a.norm_w ? nw[e] * (o[e] * inv) * silu_f(z[e]) : o[e];
+            mx = fmaxf(mx, fabsf(y));
+            a.out[a.out_tiled ? xt_off(t, c, a.VH * kD) : static_cast<int64_t>(t) * (a.VH * kD) + c] = y;
+        }
+        if (a.omax) {  // uniform
+            mx = fmaxf(mx, dpp_f<0xB1>(mx));
+            mx = fmaxf(mx, dpp_f<0x4E>(mx));
+            mx = fmaxf(mx, dpp_f<0x141>(mx));
+            mx = fmaxf(mx, dpp_f<0x140>(mx));
+            mx = fmaxf(mx, swz16_f(mx));
+            if (l32 == 0) a.omax[static_cast<int64_t>(t) * a.VH + vh] = mx;
+        }
+    }
+}
+
 // ------------------------------------------------------------------ attention prep
 // Any even rotary width: grid (T, NQ + NKV), one thread per dim.
 __global__ __launch_bounds__(256) void attn_prefill_prep_any_kernel(AttnPrefillArgs a) {
@@ -1283,6 +1482,15 @@ void gdn_prefill_carve(GdnPrefillArgs& a, float* ws) {
 }
 
 hipError_t launch_gdn_prefill(GdnPrefillArgs& a, hipStream_t s) {
+    // Few tokens: token by token in one launch (the state is read 16 bytes at a time). The scan
+    // takes about 1 us a token, 330 instructions of one wave per SIMD; the chunked kernels one
+    // chunk's 56-60 us up to 64 tokens: 1 token 55.0 / 6.1 us, 8 55.2 / 13.0, 31 56.0 / 35.5,
+    // 48 58.1 / 52.8, 64 59.7 / 68.7 (16 heads). Closer to float64, 1.4e-7 against 2.0e-7.
+    if (a.T <= kShortT && (reinterpret_cast<uintptr_t>(a.state) & 15) == 0) {
+        klaunch(gdn_short_kernel, a.VH, kShortThreads, 0, s, a);
+        if (a.VH != a.KH) klaunch(gdn_ring_kernel, blocks_for(3 * (2 * a.KH * kD + a.VH * kD)), 256, 0, s, a);
+        return hipGetLastError();
+    }
     klaunch(gdn_chunk_kernel, dim3(a.VH, a.Tp / kC), 256, 0, s, a);
     klaunch(gdn_ring_kernel, blocks_for(3 * (2 * a.KH * kD + a.VH * kD)), 256, 0, s, a);
     klaunch(gdn_state_kernel, dim3(a.VH, kD / kSW), kSThreads, 0, s, a);
