@@ -1030,11 +1030,104 @@ __global__ __launch_bounds__(256) void attn_kv_image_kernel(AttnPrefillArgs a) {
     }
 }
 
-// IMG (fp32 cache only): tiles are copied from the image attn_kv_image_kernel wrote.
+// Online softmax of one 32-key tile for the lane's query: the scores S^T[key 16 hf + 4 g4 + v]
+// become weights p[4 hf + v], (m, l) the row's running maximum and sum. Returns the factor of
+// the output so far. The reference max moves only when a score exceeds it by more than 8; a
+// row with no key yet keeps -inf and weight 0. e^y as the native 2^(y log2 e): y = score -
+// max is formed exactly, so the product's rounding moves a weight by |y| 2^-24 relative (1 ulp
+// of v_exp_f32 besides), negligible where the weights are large.
+__device__ __forceinline__ float flash_softmax(const floatx4 (&St)[2], int kv0, int qpos, int kv_end, float sc, int g4,
+                                               float& m, float& l, float (&p)[8]) {
+    float sv[8];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int key = kv0 + 16 * hf + 4 * g4 + v;
+            sv[4 * hf + v] = key <= qpos && key < kv_end ? St[hf][v] * sc : -INFINITY;
+        }
+    float tm = sv[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) tm = fmaxf(tm, sv[i]);
+    tm = fmaxf(tm, __shfl_xor(tm, 16));
+    tm = fmaxf(tm, __shfl_xor(tm, 32));
+    const float m_new = tm > m + 8.0f ? tm : m;
+    const bool live = m_new != -INFINITY;
+    const float f = live ? __builtin_amdgcn_exp2f((m - m_new) * kLog2e) : 1.0f;
+    float ps = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        p[i] = live ? __builtin_amdgcn_exp2f((sv[i] - m_new) * kLog2e) : 0.0f;
+        ps += p[i];
+    }
+    ps += __shfl_xor(ps, 16);
+    ps += __shfl_xor(ps, 32);
+    l = l * f + ps;
+    m = m_new;
+    return f;
+}
+// output rows 4 g4 + r of the wave times the factors f of lanes 4 g4 + r
+__device__ __forceinline__ void flash_rescale(float f, int g4, floatx4 (&o)[16]) {
+    if (!__any(f != 1.0f)) return;
+    float fr[4];
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) fr[rr] = __shfl(f, 4 * g4 + rr);
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+        o[t][0] *= fr[0];
+        o[t][1] *= fr[1];
+        o[t][2] *= fr[2];
+        o[t][3] *= fr[3];
+    }
+}
+
+// Epilogue of 16 rows of a block from `rbase`: o / (row sum) times the gate.
+__device__ __forceinline__ void flash_store(const AttnPrefillArgs& a, const floatx4 (&o)[16], const float (&lr)[4], int kh,
+                                            int grp, int rows, int rbase, int lane) {
+    const int r16 = lane & 15, g4 = lane >> 4;
+    // every gate value requested before the first store: the output may alias them as far as
+    // the compiler knows, and a load after a store would wait for its own round trip, 64 in a
+    // row (35 us a workgroup; 4096 tokens 762 -> 722 us)
+    float gt[4][16];
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+        const int rc = min(rbase + 4 * g4 + rr, rows - 1);  // rows past the block store nothing
+        const float* gate = a.qkv + static_cast<int64_t>(rc / grp) * a.ld_qkv +
+                            static_cast<int64_t>(kh * grp + rc % grp) * 2 * kHD + kHD;
+#pragma unroll
+        for (int tt = 0; tt < 16; ++tt) gt[rr][tt] = gate[16 * tt + r16];
+    }
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+        const int row = rbase + 4 * g4 + rr;
+        const int rc = min(row, rows - 1);
+        const int t = rc / grp, h = kh * grp + rc % grp;
+        const float inv = 1.0f / lr[rr];
+        float* out = a.out + static_cast<int64_t>(t) * (a.NQ * kHD) + static_cast<int64_t>(h) * kHD;
+        float mx = 0.0f;
+#pragma unroll
+        for (int tt = 0; tt < 16; ++tt) {
+            const int dd = 16 * tt + r16;
+            const float y = (o[tt][rr] * inv) * sigmoid_f(gt[rr][tt]);
+            mx = fmaxf(mx, fabsf(y));
+            if (row < rows) {
+                if (a.out_tiled) a.out[xt_off(t, h * kHD + dd, a.NQ * kHD)] = y;
+                else out[dd] = y;
+            }
+        }
+        if (a.omax) {  // uniform: the row's maximum over this head's 256 dims (16 lanes)
+            mx = fmaxf(mx, __shfl_xor(mx, 1));
+            mx = fmaxf(mx, __shfl_xor(mx, 2));
+            mx = fmaxf(mx, __shfl_xor(mx, 4));
+            mx = fmaxf(mx, __shfl_xor(mx, 8));
+            if (r16 == 0 && row < rows) a.omax[static_cast<int64_t>(t) * a.NQ + h] = mx;
+        }
+    }
+}
+
 // SPLIT: grid (pieces, blocks of all kv heads), else grid (blocks).
-template <bool KVB, bool IMG, bool SPLIT>
+template <bool KVB, bool SPLIT>
 __global__ __launch_bounds__(flash_waves(KVB) * 64, KVB ? 8 / flash_waves(KVB) : 1) void flash_attn_kernel(AttnPrefillArgs a) {
-    static_assert(!(KVB && IMG), "the tile image holds the parts of an fp32 cache");
     constexpr int kFW = flash_waves(KVB), kQT = 16 * kFW;
     constexpr int SS = 8 / kFW;  // staging passes (one thread's share of a tile by 512 threads each)
     constexpr int NP = KVB ? 1 : 3;  // parts of K and V
@@ -1093,11 +1186,10 @@ __global__ __launch_bounds__(flash_waves(KVB) * 64, KVB ? 8 / flash_waves(KVB) :
     // 4 g .. + 3 and 16 + 4 g .. + 3, one float2 each); split (or widened) when stored to LDS
     const int ks_row = 8 * (wave & 3) + (lane & 7), ks_c0 = 16 * (wave >> 2) + (lane >> 3);
     const int vs_g = tid & 3, vs_d = (tid >> 2) * 2;
-    float4 kst[IMG || KVB ? 1 : 4];
-    float2 vst[IMG || KVB ? 1 : 8];
+    float4 kst[KVB ? 1 : 4];
+    float2 vst[KVB ? 1 : 8];
     // (vector-typed: an array of uint4 structs here was placed in scratch memory)
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 ist[IMG ? kImgTile / (kFW * 64) : 1];
     // bf16 cache: the stored bits are the operands, K chunks as they lie, V pairs of dims
     // (8-byte aligned, as the cache rows' other accesses)
     typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
@@ -1105,13 +1197,6 @@ __global__ __launch_bounds__(flash_waves(KVB) * 64, KVB ? 8 / flash_waves(KVB) :
     uint32_t vbs[KVB ? 8 * SS : 1];
     auto vkey = [&](int j) { return vslot_key(vs_g, j); };
     auto load_tile = [&](int kv0) {
-        if constexpr (IMG) {  // tiles past the block's keys: the last one again (in the image)
-            const u32x4* src = static_cast<const u32x4*>(a.kv_img) +
-                               (static_cast<int64_t>(kh) * a.img_tiles + min(kv0, kv_end - 1) / kKT) * kImgTile;
-#pragma unroll
-            for (int j = 0; j < kImgTile / (kFW * 64); ++j) ist[j] = src[tid + kFW * 64 * j];
-            return;
-        }
         const bool live = kv0 < kv_end;
         if constexpr (KVB) {
             const uint16_t *kc = reinterpret_cast<const uint16_t*>(a.k_cache) + hoff,
@@ -1143,14 +1228,6 @@ __global__ __launch_bounds__(flash_waves(KVB) * 64, KVB ? 8 / flash_waves(KVB) :
     // Rows past the end of the keys are copies of the last one (finite): their scores are
     // masked to -inf, so their weights are exactly 0 and 0 * V adds nothing.
     auto store_tile = [&]() {
-        if constexpr (IMG) {  // the image is the two arrays' contents, chunk for chunk
-            constexpr int NJ = kImgTile / (kFW * 64);
-#pragma unroll
-            for (int j = 0; j < NJ / 2; ++j) reinterpret_cast<u32x4*>(&Kc[0][0][0][0])[tid + kFW * 64 * j] = ist[j];
-#pragma unroll
-            for (int j = 0; j < NJ / 2; ++j) reinterpret_cast<u32x4*>(&Vc[0][0][0][0])[tid + kFW * 64 * j] = ist[NJ / 2 + j];
-            return;
-        }
         if constexpr (KVB) {
 #pragma unroll
             for (int j = 0; j < 2 * SS; ++j)
@@ -1229,49 +1306,9 @@ __global__ __launch_bounds__(flash_waves(KVB) * 64, KVB ? 8 / flash_waves(KVB) :
                 }
                 St[hf] = (sb[0] + sb[1]) + (sa[0] + sa[1]);
             }
-            float sv[8];
-#pragma unroll
-            for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int key = kv0 + 16 * hf + 4 * g4 + v;
-                    sv[4 * hf + v] = key <= qpos && key < kv_end ? St[hf][v] * sc : -INFINITY;
-                }
-            float tm = sv[0];
-#pragma unroll
-            for (int i = 1; i < 8; ++i) tm = fmaxf(tm, sv[i]);
-            tm = fmaxf(tm, __shfl_xor(tm, 16));
-            tm = fmaxf(tm, __shfl_xor(tm, 32));
-            // the reference max moves only when a score exceeds it by more than 8; a row with
-            // no key yet keeps -inf and weight 0
-            const float m_new = tm > m_run + 8.0f ? tm : m_run;
-            const bool live = m_new != -INFINITY;
-            // e^y as the native 2^(y log2 e): y = score - max is formed exactly as before, so
-            // the product's rounding moves a weight by |y| 2^-24 relative (1 ulp of v_exp_f32
-            // besides), negligible where the weights are large
-            const float f = live ? __builtin_amdgcn_exp2f((m_run - m_new) * kLog2e) : 1.0f;
-            float p[8], ps = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                p[i] = live ? __builtin_amdgcn_exp2f((sv[i] - m_new) * kLog2e) : 0.0f;
-                ps += p[i];
-            }
-            ps += __shfl_xor(ps, 16);
-            ps += __shfl_xor(ps, 32);
-            l_run = l_run * f + ps;
-            m_run = m_new;
-            if (__any(f != 1.0f)) {  // rescale output rows 4 g4 + r
-                float fr[4];
-#pragma unroll
-                for (int rr = 0; rr < 4; ++rr) fr[rr] = __shfl(f, 4 * g4 + rr);
-#pragma unroll
-                for (int t = 0; t < 16; ++t) {
-                    o[t][0] *= fr[0];
-                    o[t][1] *= fr[1];
-                    o[t][2] *= fr[2];
-                    o[t][3] *= fr[3];
-                }
-            }
+            float p[8];
+            const float f = flash_softmax(St, kv0, qpos, kv_end, sc, g4, m_run, l_run, p);
+            flash_rescale(f, g4, o);
             // O[query 4 g4 + v][dim 16 t + r16] += P[query][keys] V[keys][dim], k slots
             // 8 g4 .. + 7 = keys 4 g4 .. + 3 of both halves
             bf16x8 pa[3];
@@ -1319,44 +1356,173 @@ __global__ __launch_bounds__(flash_waves(KVB) * 64, KVB ? 8 / flash_waves(KVB) :
     float lr[4];
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) lr[rr] = __shfl(l_run, 4 * g4 + rr);
-    // every gate value requested before the first store: the output may alias them as far as
-    // the compiler knows, and a load after a store would wait for its own round trip, 64 in a
-    // row (35 us a workgroup; 4096 tokens 762 -> 722 us)
-    float gt[4][16];
+    flash_store(a, o, lr, kh, grp, rows, row0 + wave * 16, lane);
+}
+
+// The same block of 128 rows of an fp32 cache from the tile image attn_kv_image_kernel wrote:
+// the same products and sums as flash_attn_kernel without an image, bit for bit. The image is
+// the LDS contents, so a tile is copied straight into LDS (global_load_lds, 16 bytes a lane)
+// with no registers in between: K of the next tile goes into a second buffer while this tile
+// is worked on, V of this tile arrives under S = K Q^T (144 KB of LDS). Against staging in 48
+// registers a thread the 4096-token attention went from 724.6 to 715.7 us in turn on one
+// board; its 825 GFLOP of bf16 part products take 578 us at the rate of a large matrix product
+// there, and the clock falls as the matrix cores fill. Ruled out: 4 waves of 32 rows (half the
+// LDS reads, but one wave a SIMD overlaps nothing: 28% slower), the next step's operands read
+// under this step's products (0.4% slower), one K array with two halves (every read waited
+// for the copy in flight: 5% slower).
+template <bool SPLIT>
+__global__ __launch_bounds__(512, 1) void flash_image_kernel(AttnPrefillArgs a) {
+    constexpr int kQT = 128, W = 8;
+    const int grp = a.NQ / a.NKV, rows = a.T * grp, nblk = (rows + kQT - 1) / kQT;
+    const int rank = SPLIT ? blockIdx.y : blockIdx.x;
+    const int qt = nblk - 1 - rank / a.NKV, kh = rank % a.NKV;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row0 = qt * kQT;
+    const int kv_end = a.pos0 + min(rows - 1, row0 + kQT - 1) / grp + 1;
+    const int piece_keys = a.piece * kKT;
+    const int kv_lo = SPLIT ? static_cast<int>(blockIdx.x) * piece_keys : 0;
+    if (SPLIT && kv_lo >= kv_end) return;  // uniform: the block has fewer pieces
+    const int kv_hi = SPLIT ? min(kv_end, kv_lo + piece_keys) : kv_end;
+    const bool whole = !SPLIT || kv_end <= piece_keys;  // the block's only piece: final output
+    const int r16 = lane & 15, g4 = lane >> 4;
+    // (separate arrays: the compiler then knows that a copy into one need not be waited for
+    // before reads of another)
+    typedef uint4 KTile[3][2][kHD / 8][16];
+    __shared__ __align__(16) KTile K0, K1;
+    __shared__ __align__(16) uint4 Vc[3][kHD / 16][4][16];
+    const float sc = 1.0f / sqrtf(static_cast<float>(kHD));
+
+    // K (half 0) or V (half 1) of a tile of the image into LDS: each wave 1 KB per instruction
+    constexpr int kCopies = kImgK / (64 * W);
+    auto copy = [&](int kv0, int half, uint4* dst) {
+        const uint4* src = static_cast<const uint4*>(a.kv_img) +
+                           (static_cast<int64_t>(kh) * a.img_tiles + min(kv0, kv_end - 1) / kKT) * kImgTile + half * kImgK;
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-        const int rc = min(row0 + wave * 16 + 4 * g4 + rr, rows - 1);  // rows past the block store nothing
-        const float* gate = a.qkv + static_cast<int64_t>(rc / grp) * a.ld_qkv +
-                            static_cast<int64_t>(kh * grp + rc % grp) * 2 * kHD + kHD;
+        for (int j = 0; j < kCopies; ++j) {
+            const int c = 64 * (W * j + wave);
+            __builtin_amdgcn_global_load_lds(
+                reinterpret_cast<const __attribute__((address_space(1))) void*>(reinterpret_cast<uintptr_t>(src + c + lane)),
+                (__attribute__((address_space(3))) void*)(dst + c), 16, 0, 0);
+        }
+    };
+    // s_waitcnt with only the vector-memory counter given: none left, or one copy's loads left
+    constexpr int kWaitAll = 0x0f70, kWaitNewestK = 0x0f70 | kCopies;
+
+    copy(kv_lo, 0, &K0[0][0][0][0]);
+    // this lane's query row, dims 32c + 8 g4 .. + 7, as three bf16 parts (the B operand)
+    const int qrow = min(row0 + wave * 16 + r16, rows - 1);
+    const int qpos = a.pos0 + qrow / grp;
+    bf16x8 qp[3][8];
+    {
+        const float* src = a.Qa + (static_cast<int64_t>(kh * grp + qrow % grp) * a.T + qrow / grp) * kHD + 8 * g4;
 #pragma unroll
-        for (int tt = 0; tt < 16; ++tt) gt[rr][tt] = gate[16 * tt + r16];
+        for (int c = 0; c < 8; ++c) {
+            const float4 x0 = *reinterpret_cast<const float4*>(src + 32 * c);
+            const float4 x1 = *reinterpret_cast<const float4*>(src + 32 * c + 4);
+            const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            uint4 p3[3];
+            split3_8(x, p3);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) qp[p][c] = __builtin_bit_cast(bf16x8, p3[p]);
+        }
     }
+    // the wave's last query position: tiles starting past it hold no key its rows attend
+    const int wlast = a.pos0 + min(row0 + wave * 16 + 15, rows - 1) / grp;
+    floatx4 o[16];  // dims 16 t + r16 of query rows 4 g4 + v
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-        const int row = row0 + wave * 16 + 4 * g4 + rr;
-        const int rc = min(row, rows - 1);
-        const int t = rc / grp, h = kh * grp + rc % grp;
-        const float inv = 1.0f / lr[rr];
-        float* out = a.out + static_cast<int64_t>(t) * (a.NQ * kHD) + static_cast<int64_t>(h) * kHD;
-        float mx = 0.0f;
+    for (int t = 0; t < 16; ++t) o[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.0f;
+
+    __builtin_amdgcn_s_waitcnt(kWaitAll);
+    lds_barrier();
+    copy(kv_lo, 1, &Vc[0][0][0][0]);
+    auto tile = [&](int kv0, const KTile& Kc, KTile& Kn) {
+        copy(kv0 + kKT, 0, &Kn[0][0][0][0]);  // past the last tile: the last one again
+        const bool live_wave = kv0 <= wlast;  // uniform per wave
+        bf16x8 pa[3];
+        // (K or P part, Q or V part) from the smallest product
+        constexpr int lo[6] = {2, 1, 0, 1, 0, 0}, ro[6] = {0, 1, 2, 0, 1, 0};
+        if (live_wave) {
+            // S^T[key 16 hf + 4 g4 + v][query r16]: the hi.hi products and the smaller part
+            // products in separate accumulators, each split over even / odd dim blocks
+            floatx4 St[2];
 #pragma unroll
-        for (int tt = 0; tt < 16; ++tt) {
-            const int dd = 16 * tt + r16;
-            const float y = (o[tt][rr] * inv) * sigmoid_f(gt[rr][tt]);
-            mx = fmaxf(mx, fabsf(y));
-            if (row < rows) {
-                if (a.out_tiled) a.out[xt_off(t, h * kHD + dd, a.NQ * kHD)] = y;
-                else out[dd] = y;
+            for (int hf = 0; hf < 2; ++hf) {
+                floatx4 sa[2], sb[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) sa[e] = sb[e] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c2 = 0; c2 < 4; ++c2) {
+                    bf16x8 kop[2][3];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+#pragma unroll
+                        for (int p = 0; p < 3; ++p)
+                            kop[e][p] = __builtin_bit_cast(bf16x8, Kc[p][hf][4 * (2 * c2 + e) + g4][r16]);
+#pragma unroll
+                    for (int i = 0; i < 6; ++i)
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            floatx4& s = i < 5 ? sb[e] : sa[e];
+                            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop[e][lo[i]], qp[ro[i]][2 * c2 + e], s, 0, 0, 0);
+                        }
+                }
+                St[hf] = (sb[0] + sb[1]) + (sa[0] + sa[1]);
+            }
+            float p[8];
+            const float f = flash_softmax(St, kv0, qpos, kv_end, sc, g4, m_run, l_run, p);
+            flash_rescale(f, g4, o);
+            uint4 p3[3];
+            split3_8(p, p3);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) pa[q] = __builtin_bit_cast(bf16x8, p3[q]);
+        }
+        // this wave's share of V is in LDS (the next K's need not be: lds_barrier would wait for
+        // it), then every wave's
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(kWaitNewestK);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        if (live_wave) {
+            // O[query 4 g4 + v][dim 16 t + r16] += P[query][keys] V[keys][dim], the part products
+            // straight into the running output
+#pragma unroll
+            for (int t2 = 0; t2 < 8; ++t2) {
+                bf16x8 vb[2][3];
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) vb[e][q] = __builtin_bit_cast(bf16x8, Vc[q][2 * t2 + e][g4][r16 ^ (4 * g4)]);
+#pragma unroll
+                for (int i = 0; i < 6; ++i)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        o[2 * t2 + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[lo[i]], vb[e][ro[i]], o[2 * t2 + e], 0, 0, 0);
             }
         }
-        if (a.omax) {  // uniform: the row's maximum over this head's 256 dims (16 lanes)
-            mx = fmaxf(mx, __shfl_xor(mx, 1));
-            mx = fmaxf(mx, __shfl_xor(mx, 2));
-            mx = fmaxf(mx, __shfl_xor(mx, 4));
-            mx = fmaxf(mx, __shfl_xor(mx, 8));
-            if (r16 == 0 && row < rows) a.omax[static_cast<int64_t>(t) * a.NQ + h] = mx;
-        }
+        __builtin_amdgcn_s_waitcnt(kWaitAll);  // this wave's share of the next K (asked for a tile ago)
+        lds_barrier();                         // every wave is done with this V, every share of the next K is in
+        copy(kv0 + kKT, 1, &Vc[0][0][0][0]);
+    };
+    for (int kv0 = kv_lo; kv0 < kv_hi; kv0 += 2 * kKT) {
+        tile(kv0, K0, K1);
+        if (kv0 + kKT < kv_hi) tile(kv0 + kKT, K1, K0);  // uniform
     }
+    __builtin_amdgcn_s_waitcnt(kWaitAll);  // nothing is on its way into LDS when the workgroup ends
+    if (!whole) {  // uniform: the piece's output and (max, sum) as they stand, lane by lane
+        const int64_t slot = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+        floatx4* po = reinterpret_cast<floatx4*>(a.part) + (slot * W + wave) * 16 * 64 + lane;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) po[64 * t] = o[t];
+        if (g4 == 0) a.part_ml[slot * kQT + wave * 16 + r16] = make_float2(m_run, l_run);
+        return;
+    }
+    float lr[4];
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) lr[rr] = __shfl(l_run, 4 * g4 + rr);
+    flash_store(a, o, lr, kh, grp, rows, row0 + wave * 16, lane);
 }
 
 // Merges the pieces of one 16-row group of a block (grid: wave groups, blocks of all kv
@@ -1566,17 +1732,17 @@ hipError_t launch_attn_prefill(const AttnPrefillArgs& in, hipStream_t s) {
         klaunch(attn_kv_image_kernel, dim3(a.img_tiles, a.NKV), 256, 0, s, a);
     }
     if (p.pieces) {
-        if (a.kv_bf16) klaunch(flash_attn_kernel<true, false, true>, grid, 64 * waves, 0, s, a);
-        else if (img) klaunch(flash_attn_kernel<false, true, true>, grid, 64 * waves, 0, s, a);
-        else klaunch(flash_attn_kernel<false, false, true>, grid, 64 * waves, 0, s, a);
+        if (a.kv_bf16) klaunch(flash_attn_kernel<true, true>, grid, 64 * waves, 0, s, a);
+        else if (img) klaunch(flash_image_kernel<true>, grid, 512, 0, s, a);
+        else klaunch(flash_attn_kernel<false, true>, grid, 64 * waves, 0, s, a);
         if (a.kv_bf16) klaunch(flash_combine_kernel<flash_waves(true)>, dim3(waves, blocks), 1024, 0, s, a, p.pieces);
         else klaunch(flash_combine_kernel<flash_waves(false)>, dim3(waves, blocks), 1024, 0, s, a, p.pieces);
     } else if (a.kv_bf16) {
-        klaunch(flash_attn_kernel<true, false, false>, grid, 64 * waves, 0, s, a);
+        klaunch(flash_attn_kernel<true, false>, grid, 64 * waves, 0, s, a);
     } else if (img) {
-        klaunch(flash_attn_kernel<false, true, false>, grid, 64 * waves, 0, s, a);
+        klaunch(flash_image_kernel<false>, grid, 512, 0, s, a);
     } else {
-        klaunch(flash_attn_kernel<false, false, false>, grid, 64 * waves, 0, s, a);
+        klaunch(flash_attn_kernel<false, false>, grid, 64 * waves, 0, s, a);
     }
     return hipGetLastError();
 }
