@@ -17,12 +17,12 @@
 //              A[i][j] = beta_i k_i.k_j e^(gamma_i - gamma_j)  (j < i)
 //              [U | W] = (I + A)^-1 [beta v | beta e^gamma k]  (forward substitution, one
 //                                                               column per thread, in registers)
-//   ring     the last three raw inputs of the block go to their ring slots (after the chunk
-//            pass, which reads the old ones).
-//   state    per (v-head, 16-column slice of the state), sequential over the chunks, on the
+//   state    per (v-head, 8-column slice of the state), sequential over the chunks, on the
 //            fp32 matrix cores: store the chunk-start state S_c, v_new = U - W S,
 //              S <- e^(gamma_last) S + K^T (e^(gamma_last - gamma) v_new)
-//            The delta rule is column-separable, so the 8 slices of a head are independent.
+//            The delta rule is column-separable, so the 16 slices of a head are independent.
+//            Then the last three raw inputs of the block go to their ring slots (the chunk
+//            pass has read the old ones).
 //   output   per (v-head, chunk), in parallel: o = e^gamma (Q S_c) + P v_new on the matrix
 //            cores, then rmsnorm_gated per (token, v-head) (src/forward_pass.cpp:86-93).
 // Causal attention, flash form on the bf16 matrix cores:
@@ -45,7 +45,8 @@ constexpr int kD = 128;   // GDN head dim
 constexpr int kC = 64;    // chunk length
 constexpr int kHD = 256;  // attention head dim
 
-// ring slots of the block's last three raw inputs
+// ring slots of the block's last three raw inputs (blocks of few tokens whose v-heads share
+// k-heads: there no workgroup is the only reader of a channel's old slots)
 __global__ __launch_bounds__(256) void gdn_ring_kernel(GdnPrefillArgs a) {
     const int KD = a.KH * kD, VD = a.VH * kD, CONV = 2 * KD + VD;
     const int t0 = a.T > 3 ? a.T - 3 : 0;
@@ -275,171 +276,194 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk_kernel(GdnPrefillArgs a) {
         col[i] = x;
         __builtin_amdgcn_sched_barrier(0);
     }
-    float* dst = (tid < kD ? a.U : a.W) + (static_cast<int64_t>(vh) * a.Tp + row0) * kD + (tid & (kD - 1));
+    __syncthreads();  // every read of A done: W takes its place, to leave in operand order
+    if (tid < kD) {
+        float* dst = a.U + (static_cast<int64_t>(vh) * a.Tp + row0) * kD + tid;
 #pragma unroll
-    for (int i = 0; i < kC; ++i) dst[static_cast<int64_t>(i) * kD] = col[i];
-    // the decayed keys of the state update, transposed: Kd[d][t] = K[t][d] e^(gamma_last - gamma_t)
-    float* kd = a.Kd + (static_cast<int64_t>(vh) * (a.Tp / kC) + c) * kD * kC;
-    for (int e = tid; e < kD * kC; e += 256) kd[e] = Ks[e & (kC - 1)][e >> 6] * edl[e & (kC - 1)];
+        for (int i = 0; i < kC; ++i) dst[static_cast<int64_t>(i) * kD] = col[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < kC; ++i) Qs[i][tid - kD] = col[i];
+    }
+    lds_barrier();
+    // operand order of the state pass (its comment): 16 bytes of lane l, step g of wave w at
+    // (8 w + g) 64 + l. W: row 16 w + l % 16, dims 16 g + 4 (l / 16) .. + 3. The decayed keys
+    // K[t][d] e^(gamma_last - gamma_t): dim 32 w + l % 32, tokens 16 (g / 2) + 8 (l / 32) + 4 (g % 2) .. + 3
+    float* wo = a.W + (static_cast<int64_t>(vh) * a.Tp + row0) * kD;
+    float* kd = a.Kd + (static_cast<int64_t>(vh) * a.Tp + row0) * kD;
+#pragma unroll
+    for (int n = 0; n < kC * kD / 4 / 256; ++n) {
+        const int f = tid + 256 * n, g = (f >> 6) & 7, w = f >> 9;
+        *reinterpret_cast<floatx4*>(wo + f * 4) = *reinterpret_cast<const floatx4*>(&Qs[16 * w + lr][16 * g + 4 * lg]);
+        const int t = 16 * (g >> 1) + 8 * (lane >> 5) + 4 * (g & 1), dd = 32 * w + (lane & 31);
+        *reinterpret_cast<floatx4*>(kd + f * 4) =
+            floatx4{Ks[t][dd] * edl[t], Ks[t + 1][dd] * edl[t + 1], Ks[t + 2][dd] * edl[t + 2], Ks[t + 3][dd] * edl[t + 3]};
+    }
 }
 
 // ------------------------------------------------------------------ GDN state scan
-constexpr int kSW = 16;         // state columns per state-scan workgroup
-constexpr int kLdSt = kD + 4;   // state slice in LDS, one row per state column (k contiguous)
-constexpr int kLdW = kD + 4;    // W rows
-constexpr int kLdKt = kC + 4;   // decayed K, transposed: one row per dim (t contiguous)
-constexpr int kLdV = kC + 4;    // v_new, transposed: one row per state column
+constexpr int kSW = 8;  // state columns per state-scan workgroup
 
-// grid (VH, 128 / kSW), 512 threads: sequential over the chunks of one state column slice.
-// Per chunk: store the chunk-start state, v_new = U - W S (written over U), then
-// S <- e^(gamma_last) S + (K e^(gamma_last - gamma))^T v_new. Two barriers per chunk:
-//   waves 0-3   v_new rows [16 w, 16 w + 16) over all 128 dims (the dim halves [0, 64) and
-//               [64, 128) in separate accumulation chains, summed in a fixed order)
-//   waves 4-7   meanwhile store the next chunk's W and decayed K (requested one chunk ago)
-//               into the other of two LDS buffers, and request the chunk after it
-//   all waves   the new state rows [16 w, 16 w + 16)
-// Operand layout: every matrix-core operand is read 16 bytes at a time. MFMA i of a 64-deep
-// product takes the reduction index 16 lg + i from lane group lg (i < 16), so a lane's
-// operands for four consecutive MFMAs are four consecutive floats of one LDS row: W rows and
-// the state slice (stored column-major) for v_new, the decayed K (transposed by the chunk
-// pass) and v_new (stored column-major) for the state update.
-constexpr int kSThreads = 512;
-__global__ __launch_bounds__(kSThreads) void gdn_state_kernel(GdnPrefillArgs a) {
-    const int vh = blockIdx.x, cs = blockIdx.y, tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6, lr = lane & 15, lg = lane >> 4;
-    const int col0 = cs * kSW;
+// v_mfma_f32_4x4x1_16b_f32, 16 blocks of D[4][4] += a[4] b[4]: lane l supplies a[l % 4] and
+// b[l % 4] of block l / 4; result register v of lane l is D[v][l % 4]. Every 2^CB consecutive
+// blocks take their a from one of them, the J-th.
+template <int CB, int J>
+__device__ __forceinline__ floatx4 mfma1(float a, float b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, CB, J, 0);
+}
+
+// four steps for both column quads: s0, s1 the state side, w the operands of steps J .. J + 3
+template <int CB, int J>
+__device__ __forceinline__ void mfma_quad(float s0, float s1, floatx4 w, floatx4 (&acc)[2]) {
+    acc[0] = mfma1<CB, J>(s0, w[0], acc[0]);
+    acc[1] = mfma1<CB, J>(s1, w[0], acc[1]);
+    acc[0] = mfma1<CB, J + 1>(s0, w[1], acc[0]);
+    acc[1] = mfma1<CB, J + 1>(s1, w[1], acc[1]);
+    acc[0] = mfma1<CB, J + 2>(s0, w[2], acc[0]);
+    acc[1] = mfma1<CB, J + 2>(s1, w[2], acc[1]);
+    acc[0] = mfma1<CB, J + 3>(s0, w[3], acc[0]);
+    acc[1] = mfma1<CB, J + 3>(s1, w[3], acc[1]);
+}
+
+__device__ __forceinline__ void swap32(float& a, float& b) {  // lanes 32-63 of a <-> lanes 0-31 of b
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
+    a = __builtin_bit_cast(float, static_cast<int>(r[0]));
+    b = __builtin_bit_cast(float, static_cast<int>(r[1]));
+}
+__device__ __forceinline__ void swap16(float& a, float& b) {  // odd 16-lane rows of a <-> even rows of b
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
+    a = __builtin_bit_cast(float, static_cast<int>(r[0]));
+    b = __builtin_bit_cast(float, static_cast<int>(r[1]));
+}
+
+// grid (VH, 128 / kSW), 256 threads: sequential over the chunks of one state column slice, on
+// the fp32 matrix cores. Per chunk: store the chunk-start state, v_new = U - W S (written over
+// U), then S <- e^(gamma_last) S + (K e^(gamma_last - gamma))^T v_new.
+//   The scan's length is fixed, so its time is that of one chunk step; with 16 v-heads 8-column
+//   slices give every compute unit a workgroup. The 4x4x1 instruction runs at the rate of
+//   16x16x4 and fills at 8 columns: the state (and v_new) is its a operand, four columns wide
+//   and broadcast over blocks, W (and the decayed K) its b operand.
+//   W and K go from memory into registers in operand order (the chunk pass lays them out so
+//   that a lane's 16 bytes are its operands of four steps and a wave's load is 1 KB in a row),
+//   two chunks ahead, each load asked for as soon as the eight products that free its registers
+//   are issued (requested together, the 32 loads of a phase made the waves wait to issue them:
+//   92 us a scan against 81); each value is used for both column quads. Only v_new and the
+//   state, 2 KB and 4 KB, pass through LDS, each with one barrier per chunk:
+//   v_new  wave w rows 16 w + lane % 16; lane group q = lane / 16 multiplies dims 16 g + 4 q + j
+//          (step g, register j), the four groups' sums are added crosswise, and lane (q, r)
+//          ends with columns 2 q, 2 q + 1 of its row
+//   state  wave w dims 32 w + lane % 32; half p = lane / 32 multiplies tokens 16 g + 8 p + 0..7,
+//          and lane (p, d) ends with columns 4 p .. + 3 of its dim, kept in registers
+// 4096 tokens of 16 heads: 134 us as 16-column slices of 16x16x4 products with W, K and U staged
+// through LDS (128 workgroups, 64 KB of LDS reads and as much of writes a chunk), 81 so; 66
+// without the loads, about 30 of it the products.
+__global__ __launch_bounds__(256, 2) void gdn_state_kernel(GdnPrefillArgs a) {
+    const int vh = blockIdx.x, col0 = blockIdx.y * kSW, tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
+    const int lr = lane & 15, q = lane >> 4;  // v_new: row of the wave's 16, lane group
+    const int d = 32 * wave + (lane & 31), p = lane >> 5;  // state: dim, half
     const int nchunk = a.Tp / kC;
-    const bool stager = wave >= 4;  // uniform per wave
-    const int st = tid & 255;       // thread index within the half
-    __shared__ __align__(16) float St[kSW][kLdSt];
-    __shared__ __align__(16) float Wl[2][kC][kLdW];
-    __shared__ __align__(16) float Kt[2][kD][kLdKt];
-    __shared__ __align__(16) float VNt[kSW][kLdV];
-    __shared__ __align__(16) float Ul[2][kC][kSW];  // the chunk's U entries of this slice
-    float* S = a.state + static_cast<int64_t>(vh) * kD * kD;
-    for (int i = tid; i < kD * kSW; i += kSThreads) St[i & 15][i >> 4] = S[(i >> 4) * kD + col0 + (i & 15)];
+    __shared__ __align__(16) float St[2][kD][4];   // the state: column quad, dim, column
+    __shared__ __align__(16) float Vn[2][kC][4];   // v_new: column quad, token, column
+    float* S = a.state + static_cast<int64_t>(vh) * kD * kD + d * kD + col0 + 4 * p;
+    floatx4 s = {S[0], S[1], S[2], S[3]};
 
-    constexpr int NF = kC * kD / 4 / 256;  // float4 of W (and of Kd) per staging thread: 8
-    floatx4 rw[NF], rk[NF], ru4;
-    auto load_chunk = [&](int c) {  // staging waves: the chunk's W, decayed K and U entries
-        const int64_t row0 = static_cast<int64_t>(c) * kC;
-        const float* W = a.W + (static_cast<int64_t>(vh) * a.Tp + row0) * kD;
-        const float* Kd = a.Kd + (static_cast<int64_t>(vh) * nchunk + c) * kD * kC;
+    floatx4 rw[2][8], rk[2][8];  // operands of two chunks
+    float2 ru[2];                // U of two chunks: this lane's two columns of its row
+    // (uniform base + 32-bit lane offset: one scalar addition moves all of a chunk's addresses)
+    const int64_t head = static_cast<int64_t>(vh) * a.Tp * kD;
+    const uint32_t ow = (wave * 512 + lane) * 4, ou = (16 * wave + lr) * kD + col0 + 2 * q, os = d * kD + col0 + 4 * p;
+    float re[2];  // e^gamma of two chunks' rows (only the last is used: a uniform address would
+                  // be a scalar load, which the next LDS wait would wait for)
+    auto chunk = [&](int c) { return head + static_cast<int64_t>(min(c, nchunk - 1)) * kC * kD; };
+    auto load_w = [&](int c, floatx4 (&r)[8], float2& u) {
+        const float* W = a.W + chunk(c);
 #pragma unroll
-        for (int i = 0; i < NF; ++i) {
-            const int f = st + 256 * i;
-            rw[i] = *reinterpret_cast<const floatx4*>(W + f * 4);
-            rk[i] = *reinterpret_cast<const floatx4*>(Kd + f * 4);
-        }
-        // U row st / 4, columns col0 + 4 (st % 4) .. + 3
-        ru4 = *reinterpret_cast<const floatx4*>(a.U + (static_cast<int64_t>(vh) * a.Tp + row0 + (st >> 2)) * kD + col0 + 4 * (st & 3));
+        for (int g = 0; g < 8; ++g) r[g] = *reinterpret_cast<const floatx4*>(W + g * 256 + ow);
+        u = *reinterpret_cast<const float2*>(a.U + chunk(c) + ou);
     };
-    auto store_chunk = [&](int b) {
+    auto load_k = [&](int c, floatx4 (&r)[8], float& e) {
+        const float* K = a.Kd + chunk(c);
 #pragma unroll
-        for (int i = 0; i < NF; ++i) {
-            const int f = st + 256 * i;
-            *reinterpret_cast<floatx4*>(&Wl[b][f >> 5][(f & 31) * 4]) = rw[i];
-            *reinterpret_cast<floatx4*>(&Kt[b][f >> 4][(f & 15) * 4]) = rk[i];
-        }
-        *reinterpret_cast<floatx4*>(&Ul[b][st >> 2][4 * (st & 3)]) = ru4;
+        for (int g = 0; g < 8; ++g) r[g] = *reinterpret_cast<const floatx4*>(K + g * 256 + ow);
+        e = a.Eg[static_cast<int64_t>(vh) * a.Tp + min(c, nchunk - 1) * kC + lane];
     };
-    // chunk 0 into buffer 0 (the staging waves), chunk 1 requested
-    if (stager) {
-        load_chunk(0);
-        store_chunk(0);
-        load_chunk(min(1, nchunk - 1));
+    load_w(0, rw[0], ru[0]);
+    load_k(0, rk[0], re[0]);
+    load_w(1, rw[1], ru[1]);
+    load_k(1, rk[1], re[1]);
+    *reinterpret_cast<floatx4*>(&St[p][d][0]) = s;
+    lds_barrier();
+    auto step = [&](int c, floatx4 (&w)[8], floatx4 (&k)[8], float2& u, float& eg) {
+        *reinterpret_cast<floatx4*>(a.Sc + (static_cast<int64_t>(vh) * nchunk + c) * kD * kD + os) = s;
+        floatx4 acc[2] = {};
+        float sa[2][8];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int g = 0; g < 8; ++g) sa[h][g] = (&St[h][0][0])[64 * g + lane];
+        const float* Wn = a.W + chunk(c + 2);
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            mfma_quad<2, 0>(sa[0][g], sa[1][g], w[g], acc);
+            w[g] = *reinterpret_cast<const floatx4*>(Wn + g * 256 + ow);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        float y[4], x[2];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            float lo = acc[0][v], hi = acc[1][v];
+            swap32(lo, hi);
+            y[v] = lo + hi;  // lanes below 32 column v, the others column 4 + v
+        }
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            swap16(y[v], y[v + 2]);
+            x[v] = y[v] + y[v + 2];
+        }
+        const float2 vn = make_float2(u.x - x[0], u.y - x[1]);
+        *reinterpret_cast<float2*>(&Vn[q >> 1][16 * wave + lr][2 * (q & 1)]) = vn;
+        *reinterpret_cast<float2*>(a.U + chunk(c) + ou) = vn;
+        u = *reinterpret_cast<const float2*>(a.U + chunk(c + 2) + ou);
+        lds_barrier();  // v_new in LDS; every read of St done
+        float va[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) va[h][g] = (&Vn[h][0][0])[64 * g + lane];
+        floatx4 e[2] = {};
+        const float elast = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, eg), 63));
+        const float* Kn = a.Kd + chunk(c + 2);
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            if (g & 1) mfma_quad<3, 4>(va[0][g >> 1], va[1][g >> 1], k[g], e);
+            else mfma_quad<3, 0>(va[0][g >> 1], va[1][g >> 1], k[g], e);
+            k[g] = *reinterpret_cast<const floatx4*>(Kn + g * 256 + ow);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            float lo = e[0][v], hi = e[1][v];
+            swap32(lo, hi);
+            s[v] = s[v] * elast + (lo + hi);
+        }
+        *reinterpret_cast<floatx4*>(&St[p][d][0]) = s;
+        eg = a.Eg[static_cast<int64_t>(vh) * a.Tp + min(c + 2, nchunk - 1) * kC + lane];
+        lds_barrier();  // the new state in LDS; every read of Vn done
+    };
+    for (int c = 0; c + 1 < nchunk; c += 2) {
+        step(c, rw[0], rk[0], ru[0], re[0]);
+        step(c + 1, rw[1], rk[1], ru[1], re[1]);
     }
-    // e^(gamma_last) of each chunk through the constant address space: scalar loads, whose
-    // waits are on the scalar / LDS counter. (A vector load of it one chunk ahead made the
-    // loop's register copy wait for every vector load in flight -- the staged chunk too --
-    // at the end of each step.)
-    typedef __attribute__((address_space(4))) const float cfloat;
-    const cfloat* eg_last = reinterpret_cast<const cfloat*>(
-        reinterpret_cast<uintptr_t>(a.Eg + static_cast<int64_t>(vh) * a.Tp + kC - 1));
-    __syncthreads();  // the state slice and chunk 0 are in LDS
-    for (int i = tid; i < kD * kSW; i += kSThreads)
-        a.Sc[static_cast<int64_t>(vh) * nchunk * kD * kD + (i >> 4) * kD + col0 + (i & 15)] = St[i & 15][i >> 4];
-    // Phase 2 of chunk c: the new state rows [16 w, 16 w + 16) -- rows 16 w + 4 lg + v of
-    // column lr in this lane -- to LDS
-    auto phase2 = [&](int b, float elast) {
-        floatx4 sn = *reinterpret_cast<const floatx4*>(&St[lr][16 * wave + 4 * lg]);
-        sn = sn * elast;
-        floatx4 ch[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+    if (nchunk & 1) step(nchunk - 1, rw[0], rk[0], ru[0], re[0]);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 ka = *reinterpret_cast<const float4*>(&Kt[b][16 * wave + lr][16 * lg + 4 * q]);
-            const float4 vv = *reinterpret_cast<const float4*>(&VNt[lr][16 * lg + 4 * q]);
-            ch[0] = mfma4(ka.x, vv.x, ch[0]);
-            ch[1] = mfma4(ka.y, vv.y, ch[1]);
-            ch[0] = mfma4(ka.z, vv.z, ch[0]);
-            ch[1] = mfma4(ka.w, vv.w, ch[1]);
-        }
-        sn = sn + (ch[0] + ch[1]);
-        *reinterpret_cast<floatx4*>(&St[lr][16 * wave + 4 * lg]) = sn;
-    };
-    // The two roles run separate loops with the same barriers; the staging waves only load
-    // from memory and the v_new waves only store (v_new, and the chunk-start states from LDS),
-    // so no wait for a load one step old also waits for the stores issued since. (One loop
-    // with a branch per role made each step wait for the previous step's stores.)
-    if (!stager) {
-        const int vb = wave;
-        for (int c = 0; c < nchunk; ++c) {
-            const int b = c & 1;
-            const float elast = eg_last[static_cast<int64_t>(c) * kC];
-            if (c > 0) {  // the chunk-start state S_c (chunk 0's went out before the loop)
-                float* Sc = a.Sc + (static_cast<int64_t>(vh) * nchunk + c) * kD * kD + col0;
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int i = tid + 256 * j, row = i >> 2, q = 4 * (i & 3);  // 16 bytes of row `row`
-                    *reinterpret_cast<float4*>(Sc + row * kD + q) =
-                        make_float4(St[q][row], St[q + 1][row], St[q + 2][row], St[q + 3][row]);
-                }
-            }
-            // v_new rows [16 w, 16 w + 16) over dims [0, 64) and [64, 128): four chains each
-            floatx4 part[2];
-#pragma unroll
-            for (int kq = 0; kq < 2; ++kq) {
-                floatx4 ch[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) ch[q] = floatx4{0.f, 0.f, 0.f, 0.f};
-                const int k0 = 64 * kq + 16 * lg;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float4 wa = *reinterpret_cast<const float4*>(&Wl[b][16 * vb + lr][k0 + 4 * q]);
-                    const float4 sb = *reinterpret_cast<const float4*>(&St[lr][k0 + 4 * q]);
-                    ch[0] = mfma4(wa.x, sb.x, ch[0]);
-                    ch[1] = mfma4(wa.y, sb.y, ch[1]);
-                    ch[2] = mfma4(wa.z, sb.z, ch[2]);
-                    ch[3] = mfma4(wa.w, sb.w, ch[3]);
-                }
-                part[kq] = (ch[0] + ch[1]) + (ch[2] + ch[3]);
-            }
-            float* U = a.U + (static_cast<int64_t>(vh) * a.Tp + static_cast<int64_t>(c) * kC) * kD + col0;
-            floatx4 x;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                x[v] = Ul[b][16 * vb + 4 * lg + v][lr] - (part[0][v] + part[1][v]);
-                U[(16 * vb + 4 * lg + v) * kD + lr] = x[v];
-            }
-            *reinterpret_cast<floatx4*>(&VNt[lr][16 * vb + 4 * lg]) = x;
-            lds_barrier();  // VNt and the next chunk's buffer written; every v_new read of St done
-            phase2(b, elast);
-            lds_barrier();  // the new state rows in LDS; every read of VNt and of buffer b done
-        }
-    } else {
-        for (int c = 0; c < nchunk; ++c) {
-            const int b = c & 1;
-            const float elast = eg_last[static_cast<int64_t>(c) * kC];
-            // chunk c + 1, requested one step ago, into the other buffer (after the last chunk:
-            // the last one again, into the buffer nothing reads any more)
-            store_chunk(b ^ 1);
-            load_chunk(min(c + 2, nchunk - 1));
-            lds_barrier();
-            phase2(b, elast);
-            lds_barrier();
-        }
+    for (int v = 0; v < 4; ++v) S[v] = s[v];
+    // ring slots of the block's last three raw inputs (the chunk pass has read the old ones)
+    const int CONV = (2 * a.KH + a.VH) * kD, t0 = a.T > 3 ? a.T - 3 : 0;
+    for (int i = (blockIdx.y * gridDim.x + vh) * 256 + tid; i < (a.T - t0) * CONV; i += gridDim.x * gridDim.y * 256) {
+        const int t = t0 + i / CONV, ch = i % CONV;
+        a.conv_ring[static_cast<int64_t>((a.pos0 + t) & 3) * CONV + ch] = a.qkv[static_cast<int64_t>(t) * a.ld_qkv + ch];
     }
-    for (int i = tid; i < kD * kSW; i += kSThreads) S[(i >> 4) * kD + col0 + (i & 15)] = St[i & 15][i >> 4];
 }
 
 // ------------------------------------------------------------------ GDN chunk output
@@ -1658,8 +1682,7 @@ hipError_t launch_gdn_prefill(GdnPrefillArgs& a, hipStream_t s) {
         return hipGetLastError();
     }
     klaunch(gdn_chunk_kernel, dim3(a.VH, a.Tp / kC), 256, 0, s, a);
-    klaunch(gdn_ring_kernel, blocks_for(3 * (2 * a.KH * kD + a.VH * kD)), 256, 0, s, a);
-    klaunch(gdn_state_kernel, dim3(a.VH, kD / kSW), kSThreads, 0, s, a);
+    klaunch(gdn_state_kernel, dim3(a.VH, kD / kSW), 256, 0, s, a);
     klaunch(gdn_out_kernel, dim3(a.VH, a.Tp / kC), 256, 0, s, a);
     return hipGetLastError();
 }
