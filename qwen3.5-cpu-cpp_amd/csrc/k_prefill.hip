@@ -65,77 +65,117 @@ __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
 }
 
 // ------------------------------------------------------------------ GDN chunk
+constexpr int kLdC = kD + 4;
+constexpr int kLdA = 20;  // rows of A's 16 x 16 blocks
+constexpr int kRun = 8;   // tokens per conv run
+
+// block (r, b) of the lower triangle of 16 x 16 blocks
+__device__ __forceinline__ constexpr int tri(int r, int b) { return r * (r + 1) / 2 + b; }
+
+// 4 x 4 transpose over the four lanes of a quad and four registers
+__device__ __forceinline__ floatx4 quad_transpose(floatx4 x, int lane) {
+    const bool o1 = lane & 1, o2 = lane & 2;
+    const float s0 = dpp_f<0xB1>(o1 ? x[0] : x[1]), s1 = dpp_f<0xB1>(o1 ? x[2] : x[3]);  // from lane ^ 1
+    x = o1 ? floatx4{s0, x[1], s1, x[3]} : floatx4{x[0], s0, x[2], s1};
+    const float t0 = dpp_f<0x4E>(o2 ? x[0] : x[2]), t1 = dpp_f<0x4E>(o2 ? x[1] : x[3]);  // from lane ^ 2
+    return o2 ? floatx4{t0, t1, x[2], x[3]} : floatx4{x[0], x[1], t0, t1};
+}
+
+// Wave WV's share of the chunk's products: Q K^T of row block WV and K K^T of row block 3 - WV,
+// five 16 x 16 blocks of the lower triangle in all. P goes to memory, A to LDS: blocks below
+// the diagonal negated, the diagonal one as T = (I + A)^-1 (column lane % 16 by substitution).
+template <int WV>
+__device__ __forceinline__ void gdn_products(const float (*Qs)[kLdC], const float (*Ks)[kLdC], float (*As)[16][kLdA],
+                                             const double* gam, const float* beta, float* P, int lane) {
+    constexpr int RK = 3 - WV, NB = (WV > RK ? WV : RK) + 1;
+    const int lr = lane & 15, lg = lane >> 4;
+    floatx4 sq[WV + 1] = {}, sk[RK + 1] = {};
+    // MFMA j of a 16-deep step takes dim 4 lg + j of lane group lg: operands 16 bytes at a time
+#pragma unroll 2
+    for (int k = 0; k < kD; k += 16) {
+        const floatx4 q = *reinterpret_cast<const floatx4*>(&Qs[16 * WV + lr][k + 4 * lg]);
+        floatx4 kb[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) kb[b] = *reinterpret_cast<const floatx4*>(&Ks[16 * b + lr][k + 4 * lg]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int b = 0; b <= WV; ++b) sq[b] = mfma4(q[j], kb[b][j], sq[b]);
+#pragma unroll
+            for (int b = 0; b <= RK; ++b) sk[b] = mfma4(kb[RK][j], kb[b][j], sk[b]);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b <= RK; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = 16 * RK + 4 * lg + v, j = 16 * b + lr;
+            const float x = j < i ? beta[i] * sk[b][v] * expf(static_cast<float>(gam[i] - gam[j])) : 0.0f;
+            As[tri(RK, b)][4 * lg + v][lr] = b < RK ? -x : x;
+        }
+#pragma unroll
+    for (int b = 0; b <= WV; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = 16 * WV + 4 * lg + v, j = 16 * b + lr;
+            P[i * kC + j] = j <= i ? sq[b][v] * expf(static_cast<float>(gam[i] - gam[j])) : 0.0f;
+        }
+    float (*D)[kLdA] = As[tri(RK, RK)];
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        x[i] = i == lr ? 1.0f : 0.0f;
+#pragma unroll
+        for (int k = 0; k < i; ++k) x[i] = fmaf(-D[i][k], x[k], x[i]);
+    }
+    if (lg == 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) D[i][lr] = x[i];
+    }
+}
+
 // grid (VH, Tp / 64), 256 threads: the whole chunk pass of one (v-head, chunk of 64 tokens).
-//   inputs   thread (run, quad) convolves channels 4 quad .. + 3 of the head's q and k over
+//   inputs   thread (run, quad) convolves channels 4 quad .. + 3 of the head's q, k and v over
 //            tokens 8 run .. + 7 of the chunk (eleven raw rows, 16 bytes per load), and each
 //            32-lane half-wave (one run) sums a token's squares for the l2norm (in double);
-//            threads 0..127 convolve v channel tid over the 64 tokens (the column they solve
-//            for below); wave 0 forms beta and g, thread 0 the cumulative sum.
-//   products P and A on the fp32 matrix cores over the lower triangle of 16 x 16 blocks
-//            (three block pairs per wave, the last wave one), K and Q rows padded to 132
-//            floats so the 16 rows x 4 dims of an operand read fall in 64 distinct banks; A
-//            takes the place of Q in LDS once the products are done (68 KB in all: two
-//            workgroups per CU).
-//   solve    threads 0..127 the columns of beta v, 128..255 those of beta e^gamma k; step i
-//            requests row i + 1 of A before it computes, so it waits once per row.
-constexpr int kLdC = kD + 4;
-constexpr int kLdA = kC + 4;  // A rows: 16-byte aligned, read four entries at a time
-constexpr int kRun = 8;       // tokens per q / k conv run
+//            wave 0 forms beta and g and their running sum (a wave scan in double).
+//   products P and A on the fp32 matrix cores over the lower triangle of 16 x 16 blocks, five
+//            blocks per wave (gdn_products); K and Q rows padded to 132 floats so that the 16
+//            rows of an operand read fall in 64 distinct banks.
+//   solve    [U | W] in 16 column groups, four per wave, block by block on the matrix cores:
+//            X_b = T_bb (R_b - sum of A_bc X_c over c < b). A product's result registers
+//            (rows 4 lg + v of column lr) are the next one's operands with its steps in the
+//            order 4 lg + j, so X stays in registers.
+// beta v takes Q's place once the products are done (80 KB of LDS: two workgroups per CU).
+// 4096 tokens of 16 heads: 115 us with the solve as substitution, one column of 64 per thread
+// (2016 dependent fused multiply-adds and 20 KB of code), one thread summing gamma and the v
+// columns convolved by half the threads; 90 so, and one chunk's passes 58 -> 43 us. Of the 90 the
+// exact SiLU divisions take 16 and the products 8; 250 MB of inputs and results take 53 at the
+// rate of a large copy.
 __global__ __launch_bounds__(256, 2) void gdn_chunk_kernel(GdnPrefillArgs a) {
     const int vh = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6, lr = lane & 15, lg = lane >> 4;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
     const int rep = a.VH / a.KH, kh = vh / rep;
     const int KD = a.KH * kD, VD = a.VH * kD, CONV = 2 * KD + VD;
     const int t0 = c * kC;
-    const int64_t row0 = t0;
     __shared__ __align__(16) float Ks[kC][kLdC];
-    __shared__ __align__(16) float QA[kC * kLdC];
-    float (*Qs)[kLdC] = reinterpret_cast<float (*)[kLdC]>(QA);
-    float (*As)[kLdA] = reinterpret_cast<float (*)[kLdA]>(QA);
+    __shared__ __align__(16) float QV[kC][kLdC];  // Q, then beta v
+    __shared__ __align__(16) float As[10][16][kLdA];
     __shared__ double gam[kC];
-    __shared__ float beta[kC], gsh[kC], edl[kC];
+    __shared__ __align__(16) float beta[kC], bex[kC], edl[kC];  // beta, beta e^gamma, e^(gamma_last - gamma)
     // raw input of block token s (s < 0: the conv ring; s >= T: a padding row, zeroed below)
     auto xin4 = [&](int s, int ch) -> float4 {
         if (s >= 0) return *reinterpret_cast<const float4*>(a.qkv + static_cast<int64_t>(min(s, a.T - 1)) * a.ld_qkv + ch);
         return *reinterpret_cast<const float4*>(a.conv_ring + static_cast<int64_t>((a.pos0 + s) & 3) * CONV + ch);
     };
-    auto xin1 = [&](int s, int ch) -> float {
-        if (s >= 0) return a.qkv[static_cast<int64_t>(min(s, a.T - 1)) * a.ld_qkv + ch];
-        return a.conv_ring[static_cast<int64_t>((a.pos0 + s) & 3) * CONV + ch];
-    };
-    // every input requested up front: q / k runs, their taps, the v column and its taps
     const int run = tid >> 5, c4 = 4 * (tid & 31);
     const int ts0 = t0 + kRun * run;
-    float4 xq[kRun + 3], xk[kRun + 3];
+    auto load_run = [&](int ch, float4 (&x)[kRun + 3], float4 (&w)[4]) {
 #pragma unroll
-    for (int j = 0; j < kRun + 3; ++j) {
-        xq[j] = xin4(ts0 - 3 + j, kh * kD + c4);
-        xk[j] = xin4(ts0 - 3 + j, KD + kh * kD + c4);
-    }
-    float4 wq[4], wk[4];
+        for (int j = 0; j < kRun + 3; ++j) x[j] = xin4(ts0 - 3 + j, ch);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        wq[e] = *reinterpret_cast<const float4*>(a.conv_w + static_cast<int64_t>(kh * kD + c4 + e) * 4);
-        wk[e] = *reinterpret_cast<const float4*>(a.conv_w + static_cast<int64_t>(KD + kh * kD + c4 + e) * 4);
-    }
-    float xv[kC + 3];
-    float4 wv = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (tid < kD) {
-        const int ch = 2 * KD + vh * kD + tid;
-#pragma unroll
-        for (int j = 0; j < kC + 3; ++j) xv[j] = xin1(t0 - 3 + j, ch);
-        wv = *reinterpret_cast<const float4*>(a.conv_w + static_cast<int64_t>(ch) * 4);
-    }
-    if (tid < kC) {
-        const int t = t0 + tid;
-        float bb = 0.0f, gg = 0.0f;
-        if (t < a.T) {
-            bb = sigmoid_f(a.b[static_cast<int64_t>(t) * a.ld_ba + vh]);
-            gg = -expf(a.A_log[vh]) * softplus_f(a.a[static_cast<int64_t>(t) * a.ld_ba + vh] + a.dt_bias[vh]);
-        }
-        beta[tid] = bb;
-        gsh[tid] = gg;
-    }
+        for (int e = 0; e < 4; ++e) w[e] = *reinterpret_cast<const float4*>(a.conv_w + static_cast<int64_t>(ch + e) * 4);
+    };
     // causal conv + SiLU of four channels over a run (the reference's 4-tap window,
     // src/qwen_forward.cpp:109-118)
     auto conv_run = [&](const float4 (&x)[kRun + 3], const float4 (&w)[4], float (&y)[kRun][4]) {
@@ -155,149 +195,135 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk_kernel(GdnPrefillArgs a) {
             }
         }
     };
+    // l2norm of each token of a run, in place (a token is one half-wave)
+    auto l2norm = [&](float (&y)[kRun][4]) {
+#pragma unroll
+        for (int j = 0; j < kRun; ++j) {
+            double ss = 0.0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ss += static_cast<double>(y[j][e]) * y[j][e];
+            ss = half_wave_sum(ss);
+            const float inv = 1.0f / sqrtf(static_cast<float>(ss) + 1e-6f);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[j][e] *= inv;
+        }
+    };
+    float4 xq[kRun + 3], xk[kRun + 3], xv[kRun + 3], wq[4], wk[4], wv[4];
+    load_run(kh * kD + c4, xq, wq);
+    load_run(KD + kh * kD + c4, xk, wk);
+    if (wave == 0) {
+        const int t = t0 + lane;
+        float bb = 0.0f, gg = 0.0f;
+        if (t < a.T) {
+            bb = sigmoid_f(a.b[static_cast<int64_t>(t) * a.ld_ba + vh]);
+            gg = -expf(a.A_log[vh]) * softplus_f(a.a[static_cast<int64_t>(t) * a.ld_ba + vh] + a.dt_bias[vh]);
+        }
+        double g = gg;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const double p = __shfl_up(g, o);
+            if (lane >= o) g += p;
+        }
+        const float eg = expf(static_cast<float>(g));
+        gam[lane] = g;
+        beta[lane] = bb;
+        bex[lane] = bb * eg;
+        edl[lane] = expf(static_cast<float>(__shfl(g, 63) - g));
+        a.Eg[static_cast<int64_t>(vh) * a.Tp + t] = eg;
+    }
+    float y[kRun][4];
     {
         // q: l2norm, scaled by DK^-1/2; to LDS and (once per k-head) to the workspace
         const bool write_q = vh % rep == 0;
         const float qs = 1.0f / sqrtf(static_cast<float>(kD));
-        float y[kRun][4];
         conv_run(xq, wq, y);
+        load_run(2 * KD + vh * kD + c4, xv, wv);  // in q's registers, for after k
+        l2norm(y);
 #pragma unroll
         for (int j = 0; j < kRun; ++j) {
-            double ss = 0.0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) ss += static_cast<double>(y[j][e]) * y[j][e];
-            ss = half_wave_sum(ss);
-            const float inv = 1.0f / sqrtf(static_cast<float>(ss) + 1e-6f);
-            float4 o = make_float4((y[j][0] * inv) * qs, (y[j][1] * inv) * qs, (y[j][2] * inv) * qs, (y[j][3] * inv) * qs);
+            float4 o = make_float4(y[j][0] * qs, y[j][1] * qs, y[j][2] * qs, y[j][3] * qs);
             if (ts0 + j >= a.T) o = make_float4(0.f, 0.f, 0.f, 0.f);
-            *reinterpret_cast<float4*>(&Qs[kRun * run + j][c4]) = o;
+            *reinterpret_cast<float4*>(&QV[kRun * run + j][c4]) = o;
             if (write_q) *reinterpret_cast<float4*>(a.Qg + (static_cast<int64_t>(kh) * a.Tp + ts0 + j) * kD + c4) = o;
         }
     }
+    conv_run(xk, wk, y);
+    l2norm(y);
+#pragma unroll
+    for (int j = 0; j < kRun; ++j) {
+        float4 o = make_float4(y[j][0], y[j][1], y[j][2], y[j][3]);
+        if (ts0 + j >= a.T) o = make_float4(0.f, 0.f, 0.f, 0.f);
+        *reinterpret_cast<float4*>(&Ks[kRun * run + j][c4]) = o;
+    }
+    conv_run(xv, wv, y);
+    lds_barrier();  // Q, K, beta and gamma in LDS
     {
-        float y[kRun][4];
-        conv_run(xk, wk, y);
-#pragma unroll
-        for (int j = 0; j < kRun; ++j) {
-            double ss = 0.0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) ss += static_cast<double>(y[j][e]) * y[j][e];
-            ss = half_wave_sum(ss);
-            const float inv = 1.0f / sqrtf(static_cast<float>(ss) + 1e-6f);
-            float4 o = make_float4(y[j][0] * inv, y[j][1] * inv, y[j][2] * inv, y[j][3] * inv);
-            if (ts0 + j >= a.T) o = make_float4(0.f, 0.f, 0.f, 0.f);
-            *reinterpret_cast<float4*>(&Ks[kRun * run + j][c4]) = o;
-        }
-    }
-    __syncthreads();  // Q, K, beta, g in LDS
-    if (tid == 0) {
-        double s = 0.0;
-        for (int i = 0; i < kC; ++i) {
-            s += static_cast<double>(gsh[i]);
-            gam[i] = s;
-        }
-    }
-    __syncthreads();
-    if (tid < kC) {
-        const int64_t r = static_cast<int64_t>(vh) * a.Tp + row0 + tid;
-        a.Eg[r] = expf(static_cast<float>(gam[tid]));
-        edl[tid] = expf(static_cast<float>(gam[kC - 1] - gam[tid]));
-    }
-    // P (j <= i) and A (j < i): Q K^T and K K^T over the 128 dims for the block pairs
-    // (row block r, column block b <= r) of this wave: (3,0) (3,1) (3,2) | (3,3) (2,0) (2,1) |
-    // (2,2) (1,0) (1,1) | (0,0); lane (lr, lg) ends with rows 16 r + 4 lg + v of column 16 b + lr
-    {
-        const int pr[3] = {wave < 2 ? 3 : wave == 2 ? 2 : 0, wave == 0 ? 3 : wave == 1 ? 2 : 1,
-                           wave == 0 ? 3 : wave == 1 ? 2 : 1};
-        const int pb[3] = {wave == 0 ? 0 : wave == 1 ? 3 : wave == 2 ? 2 : 0, wave == 0 ? 1 : 0,
-                           wave == 0 ? 2 : 1};
-        const bool three = wave < 3;
-        floatx4 sq[3], sk[3];
-#pragma unroll
-        for (int p = 0; p < 3; ++p) sq[p] = sk[p] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-        for (int k = 0; k < kD; k += 4) {
-#pragma unroll
-            for (int p = 0; p < 3; ++p) {
-                if (p > 0 && !three) break;
-                const float aq = Qs[16 * pr[p] + lr][k + lg], ak = Ks[16 * pr[p] + lr][k + lg];
-                const float bk = Ks[16 * pb[p] + lr][k + lg];
-                sq[p] = mfma4(aq, bk, sq[p]);
-                sk[p] = mfma4(ak, bk, sk[p]);
-            }
-        }
-        lds_barrier();  // every wave is done reading Q: A takes its place
-        // (P blocks above the diagonal are never read and are left unwritten)
         float* P = a.P + (static_cast<int64_t>(vh) * (a.Tp / kC) + c) * kC * kC;
-#pragma unroll
-        for (int p = 0; p < 3; ++p) {
-            if (p > 0 && !three) break;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = 16 * pr[p] + 4 * lg + v;
-                const int j = 16 * pb[p] + lr;
-                const float dec = j <= i ? expf(static_cast<float>(gam[i] - gam[j])) : 0.0f;
-                P[i * kC + j] = j <= i ? sq[p][v] * dec : 0.0f;
-                As[i][j] = j < i ? beta[i] * sk[p][v] * dec : 0.0f;
-            }
-        }
+        // (P blocks above the diagonal are never read and are left unwritten)
+        if (wave == 0) gdn_products<0>(QV, Ks, As, gam, beta, P, lane);
+        else if (wave == 1) gdn_products<1>(QV, Ks, As, gam, beta, P, lane);
+        else if (wave == 2) gdn_products<2>(QV, Ks, As, gam, beta, P, lane);
+        else gdn_products<3>(QV, Ks, As, gam, beta, P, lane);
     }
-    __syncthreads();
-    // forward substitution on [beta v | beta e^gamma k], one column per thread
-    float col[kC];
-    if (tid < kD) {
+    lds_barrier();  // A in LDS; every read of Q done
 #pragma unroll
-        for (int i = 0; i < kC; ++i) {
-            float acc = 0.0f;
-            acc += wv.x * xv[i];
-            acc += wv.y * xv[i + 1];
-            acc += wv.z * xv[i + 2];
-            acc += wv.w * xv[i + 3];
-            const float v = t0 + i < a.T ? silu_f(acc) : 0.0f;
-            col[i] = beta[i] * v;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < kC; ++i) col[i] = beta[i] * expf(static_cast<float>(gam[i])) * Ks[i][tid - kD];
-    }
-    float4 ar[2][16];
-    ar[1][0] = *reinterpret_cast<const float4*>(&As[1][0]);
-#pragma unroll
-    for (int i = 1; i < kC; ++i) {
-        if (i + 1 < kC) {
-#pragma unroll
-            for (int q = 0; q < 16; ++q)
-                if (4 * q < i + 1) ar[(i + 1) & 1][q] = *reinterpret_cast<const float4*>(&As[i + 1][4 * q]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        float x = col[i];
-#pragma unroll
-        for (int k = 0; k < i; ++k) x = fmaf(-ar[i & 1][k >> 2][k & 3], col[k], x);
-        col[i] = x;
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    __syncthreads();  // every read of A done: W takes its place, to leave in operand order
-    if (tid < kD) {
-        float* dst = a.U + (static_cast<int64_t>(vh) * a.Tp + row0) * kD + tid;
-#pragma unroll
-        for (int i = 0; i < kC; ++i) dst[static_cast<int64_t>(i) * kD] = col[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < kC; ++i) Qs[i][tid - kD] = col[i];
+    for (int j = 0; j < kRun; ++j) {
+        const float b = beta[kRun * run + j];
+        float4 o = make_float4(b * y[j][0], b * y[j][1], b * y[j][2], b * y[j][3]);
+        if (ts0 + j >= a.T) o = make_float4(0.f, 0.f, 0.f, 0.f);
+        *reinterpret_cast<float4*>(&QV[kRun * run + j][c4]) = o;
     }
     lds_barrier();
-    // operand order of the state pass (its comment): 16 bytes of lane l, step g of wave w at
-    // (8 w + g) 64 + l. W: row 16 w + l % 16, dims 16 g + 4 (l / 16) .. + 3. The decayed keys
-    // K[t][d] e^(gamma_last - gamma_t): dim 32 w + l % 32, tokens 16 (g / 2) + 8 (l / 32) + 4 (g % 2) .. + 3
-    float* wo = a.W + (static_cast<int64_t>(vh) * a.Tp + row0) * kD;
-    float* kd = a.Kd + (static_cast<int64_t>(vh) * a.Tp + row0) * kD;
+    // [U | W] = (I + A)^-1 [beta v | beta e^gamma k]: waves 0 and 1 the columns of U, 2 and 3 of W
+    const int64_t head = (static_cast<int64_t>(vh) * a.Tp + t0) * kD;
+    floatx4 at[10];
+#pragma unroll
+    for (int n = 0; n < 10; ++n) at[n] = *reinterpret_cast<const floatx4*>(&As[n][lr][4 * lg]);
+    const bool isw = wave >= 2;
+    const int g0 = 4 * (wave & 1);  // first of the wave's four column groups
+    const float (*R)[kLdC] = isw ? Ks : QV;
+    floatx4 x[4][4];  // [block][column group]
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const floatx4 f = isw ? *reinterpret_cast<const floatx4*>(&bex[16 * b + 4 * lg]) : floatx4{1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) x[b][g][v] = f[v] * R[16 * b + 4 * lg + v][16 * (g0 + g) + lr];
+#pragma unroll
+        for (int e = 0; e < b; ++e)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) x[b][g] = mfma4(at[tri(b, e)][j], x[e][g][j], x[b][g]);
+        floatx4 y4[4] = {};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) y4[g] = mfma4(at[tri(b, b)][j], x[b][g][j], y4[g]);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            x[b][g] = y4[g];
+            if (isw) {
+                // operand order of the state pass (its comment): row 16 b + r, dims 16 g + 4 q .. + 3 at
+                // 16-byte slot (8 b + g) 64 + 16 q + r
+                const int q = lr >> 2, r = 4 * lg + (lr & 3);
+                *reinterpret_cast<floatx4*>(a.W + head + ((8 * b + g0 + g) * 64 + 16 * q + r) * 4) = quad_transpose(y4[g], lane);
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) a.U[head + (16 * b + 4 * lg + v) * kD + 16 * (g0 + g) + lr] = y4[g][v];
+            }
+        }
+    }
+    // the decayed keys K[t][d] e^(gamma_last - gamma_t) in operand order: dim 32 w + l % 32,
+    // tokens 16 (g / 2) + 8 (l / 32) + 4 (g % 2) .. + 3 at slot (8 w + g) 64 + l
 #pragma unroll
     for (int n = 0; n < kC * kD / 4 / 256; ++n) {
         const int f = tid + 256 * n, g = (f >> 6) & 7, w = f >> 9;
-        *reinterpret_cast<floatx4*>(wo + f * 4) = *reinterpret_cast<const floatx4*>(&Qs[16 * w + lr][16 * g + 4 * lg]);
-        const int t = 16 * (g >> 1) + 8 * (lane >> 5) + 4 * (g & 1), dd = 32 * w + (lane & 31);
-        *reinterpret_cast<floatx4*>(kd + f * 4) =
-            floatx4{Ks[t][dd] * edl[t], Ks[t + 1][dd] * edl[t + 1], Ks[t + 2][dd] * edl[t + 2], Ks[t + 3][dd] * edl[t + 3]};
+        const int t = 16 * (g >> 1) + 8 * (lane >> 5) + 4 * (g & 1), d = 32 * w + (lane & 31);
+        const floatx4 e = *reinterpret_cast<const floatx4*>(&edl[t]);
+        *reinterpret_cast<floatx4*>(a.Kd + head + f * 4) =
+            floatx4{Ks[t][d] * e[0], Ks[t + 1][d] * e[1], Ks[t + 2][d] * e[2], Ks[t + 3][d] * e[3]};
     }
 }
 
@@ -631,7 +657,7 @@ __device__ __forceinline__ float rowgroup8_sum(float v) {
     return __builtin_bit_cast(float, static_cast<int>(r[0])) + __builtin_bit_cast(float, static_cast<int>(r[1]));
 }
 
-constexpr int kShortT = 48;      // most tokens
+constexpr int kShortT = 36;      // most tokens
 constexpr int kShortRun = 4;     // tokens per conv run
 constexpr int kShortThreads = 512;
 
@@ -644,7 +670,7 @@ constexpr int kShortThreads = 512;
 //          4 (l % 8) .. + 3 (as gdn_wave_kernel); the readout takes v's place in LDS
 //   out    each half-wave one token: the gated rmsnorm (or the raw readout), row maximum
 // The chunked kernels take the time of one chunk of 64 however few tokens there are, most of
-// it serial latency; a 32-token prompt of the 0.8B shape went from 3.59 to 3.11 ms.
+// it serial latency (43 us).
 __global__ __launch_bounds__(kShortThreads) void gdn_short_kernel(GdnPrefillArgs a) {
     const int vh = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int rep = a.VH / a.KH, kh = vh / rep;
@@ -1674,8 +1700,9 @@ void gdn_prefill_carve(GdnPrefillArgs& a, float* ws) {
 hipError_t launch_gdn_prefill(GdnPrefillArgs& a, hipStream_t s) {
     // Few tokens: token by token in one launch (the state is read 16 bytes at a time). The scan
     // takes about 1 us a token, 330 instructions of one wave per SIMD; the chunked kernels one
-    // chunk's 56-60 us up to 64 tokens: 1 token 55.0 / 6.1 us, 8 55.2 / 13.0, 31 56.0 / 35.5,
-    // 48 58.1 / 52.8, 64 59.7 / 68.7 (16 heads). Closer to float64, 1.4e-7 against 2.0e-7.
+    // chunk's 43 us up to 64 tokens: 6.1 us for 1 token, 20.3 for 16, 35.8 for 32, 40.5 for 36,
+    // 44.0 for 40, 52.0 for 48 (16 heads; 42.3 for 36 with two v-heads per k-head). Closer to
+    // float64, 1.4e-7 against 2.0e-7.
     if (a.T <= kShortT && (reinterpret_cast<uintptr_t>(a.state) & 15) == 0) {
         klaunch(gdn_short_kernel, a.VH, kShortThreads, 0, s, a);
         if (a.VH != a.KH) klaunch(gdn_ring_kernel, blocks_for(3 * (2 * a.KH * kD + a.VH * kD)), 256, 0, s, a);
