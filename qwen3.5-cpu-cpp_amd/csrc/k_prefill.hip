@@ -15,8 +15,8 @@
 //            Q K^T and K K^T on the fp32 matrix cores (the 10 lower-triangle 16 x 16 blocks);
 //              P[i][j] = q_i.k_j e^(gamma_i - gamma_j)      (j <= i)
 //              A[i][j] = beta_i k_i.k_j e^(gamma_i - gamma_j)  (j < i)
-//              [U | W] = (I + A)^-1 [beta v | beta e^gamma k]  (forward substitution, one
-//                                                               column per thread, in registers)
+//              [U | W] = (I + A)^-1 [beta v | beta e^gamma k]  (by 16-row blocks on the
+//                                                               matrix cores)
 //   state    per (v-head, 8-column slice of the state), sequential over the chunks, on the
 //            fp32 matrix cores: store the chunk-start state S_c, v_new = U - W S,
 //              S <- e^(gamma_last) S + K^T (e^(gamma_last - gamma) v_new)
@@ -29,10 +29,11 @@
 //   prep     q_norm + RoPE of every query row (head-major), k_norm + RoPE of every key and
 //            the values appended to the KV cache at pos0 + t (angles in double; a bf16 cache
 //            stores them rounded to nearest even and the flash kernel widens them back).
-//   flash    grid (query tiles of 128, NQ): 8 waves of 16 query rows with their q in
-//            registers (as three bf16 parts); 32-position K / V tiles in LDS (split into
-//            bf16 parts when staged); S = Q K^T and O += P V on the bf16 matrix cores from
-//            six part products each; running max / sum per row; epilogue O / l * sigmoid(gate).
+//   flash    per block of 128 (bf16 cache: 64) rows, a row one (token, head of the group):
+//            waves of 16 rows with their q in registers (as three bf16 parts); 32-position
+//            K / V tiles in LDS (in bf16 parts); S = Q K^T and O += P V on the bf16 matrix
+//            cores from six part products each; running max / sum per row; epilogue
+//            O / l * sigmoid(gate). Long key ranges are cut and merged (flash_plan).
 #include <math.h>
 
 #include "dev_common.hpp"

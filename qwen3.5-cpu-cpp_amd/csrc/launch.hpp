@@ -243,8 +243,8 @@ struct GdnPrefillArgs {
     float *conv_ring, *state;
     float* out;        // [T][VH * 128]
     // workspace (head-major, padded to Tp rows): Qg the normalised, scaled q; Eg = e^gamma
-    // of each row, gamma the chunk-local cumulative decay; Kd = K e^(gamma_last - gamma) per
-    // (v-head, chunk), transposed ([128 dims][64 rows]); P the chunk's decayed Q K^T
+    // of each row, gamma the chunk-local cumulative decay; W and Kd = K e^(gamma_last - gamma)
+    // per (v-head, chunk) in the state pass's operand order; P the chunk's decayed Q K^T
     float *Qg, *U, *W, *Eg, *Kd, *P;
     float* Sc;         // [VH][Tp / 64][128][128] state at the start of each chunk
     float* omax = nullptr;  // maximum |out| of each (token, v-head): [T][VH] (may be null)
