@@ -383,7 +383,7 @@ uint64_t attn_prefill_image_bytes(const q35_attn_prefill_args& g) {
 // partial outputs of the key ranges, where the kernel would split them
 int attn_prefill_slots(const q35_attn_prefill_args& g) {
     if (g.kv_heads <= 0 || g.q_heads % g.kv_heads != 0 || g.pos0 < 0) return 0;
-    return q35k::flash_plan(g.n_tokens, g.q_heads, g.kv_heads, g.pos0, g.kv_dtype == 1).slots;
+    return q35k::flash_plan(g.n_tokens, g.q_heads, g.kv_heads, g.pos0, g.kv_dtype == 1, q35k::device_cu_count()).slots;
 }
 }  // namespace
 
@@ -439,11 +439,8 @@ q35_status q35_attn_prefill(const q35_attn_prefill_args* args, q35_stream s) {
         a.kv_img = a.Qa + used / 4;
         used += img;
     }
-    const int slots = attn_prefill_slots(g);
-    if (slots && g.workspace_bytes >= used + static_cast<uint64_t>(q35k::attn_prefill_part_floats(slots)) * 4) {
-        a.part = a.Qa + used / 4;
-        a.part_slots = slots;
-    }
+    a.part_slots = static_cast<int>(q35k::attn_prefill_part_room(static_cast<int64_t>((g.workspace_bytes - used) / 4)));
+    if (a.part_slots) a.part = a.Qa + used / 4;
     a.out = g.out;
     return launched(q35k::launch_attn_prefill(a, as_stream(s)), "q35_attn_prefill");
 }

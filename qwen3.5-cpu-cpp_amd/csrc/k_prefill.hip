@@ -979,12 +979,6 @@ __global__ __launch_bounds__(256) void attn_prefill_prep_kernel(AttnPrefillArgs 
 }
 
 // ------------------------------------------------------------------ flash attention
-// waves per workgroup, 16 query rows each: with a bf16 cache two workgroups of 4 share a
-// compute unit, and one's staging and barriers run under the other's products
-constexpr int kBf16Waves = 4;
-constexpr int flash_waves(bool kv_bf16) { return kv_bf16 ? kBf16Waves : 8; }
-constexpr int kKT = 32;           // keys per tile
-constexpr int kFlashPieces = 128;  // most pieces of a block
 constexpr float kLog2e = 1.44269504088896341f;
 
 // 128 query rows per workgroup (16 per wave), causal, keys of earlier blocks from the cache,
@@ -1722,47 +1716,8 @@ int64_t attn_prefill_image_floats(int NKV, int pos0, int T) {
 }
 
 int64_t attn_prefill_part_floats(int slots) { return static_cast<int64_t>(slots) * 16 * (kHD + 2); }
-
-// Cuts blocks into pieces where the longest block would outlast an even share of the work.
-// All times in tiles of 32 keys (5.9 us a tile of an fp32 cache, 3.1 us of a bf16 one). One
-// workgroup runs per compute unit and they start longest first, so unsplit blocks take the
-// longest of them or, with more blocks than compute units, the longest pair that shares one.
-// Pieces of c tiles that all start at once take c and about one more for the query rows and
-// the stores; more of them take an even share and about half a piece of unevenness. The merge
-// and its launch are about four more, and a hundredth per piece for its 128 KB of partial
-// output. Split when that is a tenth less. Blocks of up to 64 tiles (2048 keys) stay whole:
-// their output keeps the same bits whatever workspace the caller gives.
-FlashPlan flash_plan(int T, int NQ, int NKV, int pos0, bool kv_bf16) {
-    const FlashPlan whole{0, 0, 0};
-    const int waves = flash_waves(kv_bf16), kQT = 16 * waves;
-    const int grp = NQ / NKV, rows = T * grp, nblk = (rows + kQT - 1) / kQT;
-    const int64_t items = static_cast<int64_t>(nblk) * NKV;
-    const int cu = device_cu_count() * (8 / waves);  // workgroups that run at once
-    // tiles of block b; rank r (longest first) is block nblk - 1 - r / NKV
-    const auto tiles = [&](int64_t b) {
-        return static_cast<int>((pos0 + std::min<int64_t>(rows - 1, b * kQT + kQT - 1) / grp) / kKT + 1);
-    };
-    const int most = tiles(nblk - 1);
-    if (most <= 64 || items >= 2 * cu) return whole;
-    const auto ranked = [&](int64_t r) { return r < items ? tiles(nblk - 1 - r / NKV) : 0; };
-    double best = most;
-    for (int i = 0; i < cu && cu + i < items; ++i) best = std::max<double>(best, ranked(cu - 1 - i) + ranked(cu + i));
-    best *= 0.9;
-    FlashPlan p = whole;
-    for (int pieces = 2; pieces <= kFlashPieces && pieces * items * waves <= kFlashSlots; ++pieces) {
-        const int c = (most + pieces - 1) / pieces;
-        int64_t n = 0, all = 0;
-        for (int b = 0; b < nblk; ++b) {
-            n += static_cast<int64_t>((tiles(b) + c - 1) / c) * NKV;
-            all += static_cast<int64_t>(tiles(b)) * NKV;
-        }
-        const double t = (n <= cu ? c + 1.0 : static_cast<double>(all + n) / cu + 0.6 * c) + 4.0 + 0.01 * n;
-        if (t < best) {
-            best = t;
-            p = FlashPlan{c, (most + c - 1) / c, static_cast<int>((most + c - 1) / c * items * waves)};
-        }
-    }
-    return p;
+int64_t attn_prefill_part_room(int64_t floats) {
+    return std::min<int64_t>(std::max<int64_t>(floats, 0) / (16 * (kHD + 2)), kFlashSlots);
 }
 
 hipError_t launch_attn_prefill(const AttnPrefillArgs& in, hipStream_t s) {
@@ -1771,9 +1726,8 @@ hipError_t launch_attn_prefill(const AttnPrefillArgs& in, hipStream_t s) {
     else klaunch(attn_prefill_prep_any_kernel, dim3(a.T, a.NQ + a.NKV), 256, 0, s, a);
     const int waves = flash_waves(a.kv_bf16), kQT = 16 * waves;
     const int blocks = (a.T * (a.NQ / a.NKV) + kQT - 1) / kQT * a.NKV;
-    FlashPlan p{0, 0, 0};
-    if (a.part) p = flash_plan(a.T, a.NQ, a.NKV, a.pos0, a.kv_bf16);
-    if (p.slots > a.part_slots) p = FlashPlan{0, 0, 0};
+    FlashPlan p{};
+    if (a.part) p = flash_plan(a.T, a.NQ, a.NKV, a.pos0, a.kv_bf16, device_cu_count(), a.part_slots);
     a.piece = p.piece;
     a.part_ml = p.pieces ? reinterpret_cast<float2*>(a.part + static_cast<int64_t>(p.slots) * 16 * kHD) : nullptr;
     const dim3 grid = p.pieces ? dim3(p.pieces, blocks) : dim3(blocks);

@@ -7,6 +7,8 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "plans.hpp"
+
 namespace q35k {
 
 // Per-launch timing of a host thread. While launch_timer() is set, every launch records the
@@ -276,21 +278,16 @@ struct AttnPrefillArgs {
     void* kv_img = nullptr;
     int img_tiles = 0;  // set by the launch
     // optional: attn_prefill_part_floats(part_slots) floats, 16-byte aligned, for the partial
-    // outputs of key ranges (flash_plan; without them no block is split)
+    // outputs of key ranges (flash_plan, which cuts into at most part_slots; without them no
+    // block is split)
     float* part = nullptr;
     int part_slots = 0;
     int piece = 0;               // set by the launch: tiles of 32 keys per workgroup
     float2* part_ml = nullptr;   // set by the launch: (max, sum) of each slot's 16 rows
 };
-// How the attention kernel splits a block of T tokens at pos0 over key ranges: tiles per piece,
-// pieces of the longest row block (0: not split) and the partial outputs of 16 rows ("slots")
-// that takes, at most kFlashSlots (135 MB).
-struct FlashPlan {
-    int piece, pieces, slots;
-};
-constexpr int kFlashSlots = 8192;
-FlashPlan flash_plan(int T, int NQ, int NKV, int pos0, bool kv_bf16);
 int64_t attn_prefill_part_floats(int slots);
+// slots that `floats` floats have room for
+int64_t attn_prefill_part_room(int64_t floats);
 int64_t attn_prefill_workspace_floats(int NQ, int T);
 int attn_prefill_image_tiles(int pos0, int T);
 int64_t attn_prefill_image_floats(int NKV, int pos0, int T);

@@ -1,0 +1,70 @@
+#pragma once
+// How prefill kernels cut their work: functions of sizes alone (no GPU types), so that the
+// rules can be checked on any host.
+#include <algorithm>
+#include <cstdint>
+
+namespace q35k {
+
+// ---------------------------------------------------------------- key ranges of the attention prefill
+// waves per workgroup, 16 query rows each: with a bf16 cache two workgroups of 4 share a
+// compute unit, and one's staging and barriers run under the other's products
+constexpr int kBf16Waves = 4;
+constexpr int flash_waves(bool kv_bf16) { return kv_bf16 ? kBf16Waves : 8; }
+constexpr int kKT = 32;             // keys per tile
+constexpr int kFlashPieces = 128;   // most pieces of a block
+constexpr int kFlashSlots = 8192;   // most partial outputs ("slots": 16 rows of one piece; 135 MB)
+constexpr int kFlashWhole = 64;     // blocks of up to so many tiles are never cut
+
+// How the attention kernel splits a block of T tokens at pos0 over key ranges: tiles per piece,
+// pieces of the longest row block (0: not split), the slots that takes, and the expected time
+// (in tiles; 0 where no split is considered).
+struct FlashPlan {
+    int piece, pieces, slots;
+    double time;
+};
+
+// Cuts blocks into pieces where the longest block would outlast an even share of the work, into
+// at most `room` slots on `n_cu` compute units.
+// All times in tiles of 32 keys (5.9 us a tile of an fp32 cache, 3.1 us of a bf16 one). One
+// workgroup runs per compute unit and they start longest first, so unsplit blocks take the
+// longest of them or, with more blocks than compute units, the longest pair that shares one.
+// Pieces of c tiles that all start at once take c and about one more for the query rows and
+// the stores; more of them take an even share and about half a piece of unevenness. The merge
+// and its launch are about four more, and a hundredth per piece for its 128 KB of partial
+// output. Split when that is a tenth less. Blocks of up to 64 tiles (2048 keys) stay whole:
+// their output keeps the same bits whatever workspace the caller gives.
+inline FlashPlan flash_plan(int T, int NQ, int NKV, int pos0, bool kv_bf16, int n_cu, int64_t room = kFlashSlots) {
+    const int waves = flash_waves(kv_bf16), kQT = 16 * waves;
+    const int grp = NQ / NKV, rows = T * grp, nblk = (rows + kQT - 1) / kQT;
+    const int64_t items = static_cast<int64_t>(nblk) * NKV;
+    const int cu = n_cu * (8 / waves);  // workgroups that run at once
+    room = std::min<int64_t>(room, kFlashSlots);
+    // tiles of block b; rank r (longest first) is block nblk - 1 - r / NKV
+    const auto tiles = [&](int64_t b) {
+        return static_cast<int>((pos0 + std::min<int64_t>(rows - 1, b * kQT + kQT - 1) / grp) / kKT + 1);
+    };
+    FlashPlan p{0, 0, 0, 0.0};
+    const int most = tiles(nblk - 1);
+    if (most <= kFlashWhole || items >= 2 * cu) return p;
+    const auto ranked = [&](int64_t r) { return r < items ? tiles(nblk - 1 - r / NKV) : 0; };
+    p.time = most;
+    for (int i = 0; i < cu && cu + i < items; ++i) p.time = std::max<double>(p.time, ranked(cu - 1 - i) + ranked(cu + i));
+    double best = 0.9 * p.time;
+    for (int pieces = 2; pieces <= kFlashPieces && pieces * items * waves <= room; ++pieces) {
+        const int c = (most + pieces - 1) / pieces;
+        int64_t n = 0, all = 0;
+        for (int b = 0; b < nblk; ++b) {
+            n += static_cast<int64_t>((tiles(b) + c - 1) / c) * NKV;
+            all += static_cast<int64_t>(tiles(b)) * NKV;
+        }
+        const double t = (n <= cu ? c + 1.0 : static_cast<double>(all + n) / cu + 0.6 * c) + 4.0 + 0.01 * n;
+        if (t < best) {
+            best = t;
+            p = FlashPlan{c, (most + c - 1) / c, static_cast<int>((most + c - 1) / c * items * waves), t};
+        }
+    }
+    return p;
+}
+
+}  // namespace q35k
