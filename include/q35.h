@@ -403,10 +403,10 @@ q35_status q35_gdn_prefill(const q35_gdn_prefill_args *args, q35_stream s);
  * attention kernel's tile layout (3 KB per position and kv head), and, for few tokens on
  * more than 2048 positions, the partial outputs of key ranges that run in parallel (up to
  * 135 MB). A workspace of at least NQ * n * HD * 4 + 256 bytes but smaller than that is
- * accepted: without room for the tiles the kernel splits every tile itself (slower, same
- * results), with room for some of the partial outputs it cuts the keys into as many ranges as
- * fit, and without any it walks all keys of a block in one workgroup (slower, the same results
- * to fp32 rounding). Requires HD == 256. */
+ * accepted: without room for the tiles, or where cutting the keys gains more with it, the kernel
+ * splits every tile itself (slower, same results); with room for some of the partial outputs it
+ * cuts the keys into fewer ranges, and without any it walks all keys of a block in one workgroup
+ * (slower, the same results to fp32 rounding). Requires HD == 256. */
 typedef struct q35_attn_prefill_args {
     int32_t n_tokens, pos0, q_heads, kv_heads, head_dim, rotary_dim;
     int32_t kv_dtype;      /* cache elements: 0 = fp32, 1 = bf16 (as q35_attn_decode_args) */

@@ -431,16 +431,7 @@ q35_status q35_attn_prefill(const q35_attn_prefill_args* args, q35_stream s) {
     a.k_cache = g.k_cache;
     a.v_cache = g.v_cache;
     a.kv_bf16 = g.kv_dtype == 1;
-    a.Qa = static_cast<float*>(g.workspace);
-    // what the workspace has room for: the pre-split tiles first, then the partial outputs
-    uint64_t used = attn_prefill_min_bytes(g);
-    const uint64_t img = attn_prefill_image_bytes(g);
-    if (img && g.workspace_bytes >= used + img) {
-        a.kv_img = a.Qa + used / 4;
-        used += img;
-    }
-    a.part_slots = static_cast<int>(q35k::attn_prefill_part_room(static_cast<int64_t>((g.workspace_bytes - used) / 4)));
-    if (a.part_slots) a.part = a.Qa + used / 4;
+    q35k::attn_prefill_carve(a, static_cast<float*>(g.workspace), static_cast<int64_t>(g.workspace_bytes / 4));
     a.out = g.out;
     return launched(q35k::launch_attn_prefill(a, as_stream(s)), "q35_attn_prefill");
 }

@@ -1036,8 +1036,7 @@ __device__ __forceinline__ void split3_8(const float (&x)[8], uint4 (&c)[3]) {
 
 // The flash kernel's LDS image of one 32-key tile of an fp32 cache: K chunks Kc[3][2][32][16]
 // then V chunks Vc[3][16][4][16] (the layouts described at that kernel), 16-byte chunks.
-constexpr int kImgK = 3 * 2 * (kHD / 8) * 16;
-constexpr int kImgTile = 2 * kImgK;
+static_assert(kImgK == 3 * 2 * (kHD / 8) * 16, "K chunks of a tile");
 // key of slot 8 g + j of a V chunk: keys 4 g .. + 3 of the tile's first half, then the same
 // four of its second half
 __device__ __forceinline__ int vslot_key(int g, int j) { return (j < 4 ? 0 : 12) + 4 * g + j; }
@@ -1183,7 +1182,7 @@ __global__ __launch_bounds__(flash_waves(KVB) * 64, KVB ? 8 / flash_waves(KVB) :
     const int row0 = qt * kQT;
     // keys of the block, and this workgroup's piece of them
     const int kv_end = a.pos0 + min(rows - 1, row0 + kQT - 1) / grp + 1;
-    const int piece_keys = a.piece * kKT;
+    const int piece_keys = a.plan.piece * kKT;
     const int kv_lo = SPLIT ? static_cast<int>(blockIdx.x) * piece_keys : 0;
     if (SPLIT && kv_lo >= kv_end) return;  // uniform: the block has fewer pieces
     const int kv_hi = SPLIT ? min(kv_end, kv_lo + piece_keys) : kv_end;
@@ -1425,7 +1424,7 @@ __global__ __launch_bounds__(512, 1) void flash_image_kernel(AttnPrefillArgs a) 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row0 = qt * kQT;
     const int kv_end = a.pos0 + min(rows - 1, row0 + kQT - 1) / grp + 1;
-    const int piece_keys = a.piece * kKT;
+    const int piece_keys = a.plan.piece * kKT;
     const int kv_lo = SPLIT ? static_cast<int>(blockIdx.x) * piece_keys : 0;
     if (SPLIT && kv_lo >= kv_end) return;  // uniform: the block has fewer pieces
     const int kv_hi = SPLIT ? min(kv_end, kv_lo + piece_keys) : kv_end;
@@ -1585,7 +1584,7 @@ __global__ __launch_bounds__(1024) void flash_combine_kernel(AttnPrefillArgs a, 
     const int r16 = lane & 15, g4 = lane >> 4;
     const int row0 = qt * QT + 16 * group;
     const int kv_end = a.pos0 + min(rows - 1, qt * QT + QT - 1) / grp + 1;
-    const int n = (kv_end + a.piece * kKT - 1) / (a.piece * kKT);
+    const int n = (kv_end + a.plan.piece * kKT - 1) / (a.plan.piece * kKT);
     if (n <= 1 || row0 >= rows) return;  // uniform: already final, or no rows
     __shared__ __align__(16) float f_s[kFlashPieces][16];
     __shared__ float red[64][17], mred[16][16];
@@ -1709,15 +1708,20 @@ hipError_t launch_gdn_prefill(GdnPrefillArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-int64_t attn_prefill_workspace_floats(int NQ, int T) { return static_cast<int64_t>(NQ) * T * kHD + 64; }
-int attn_prefill_image_tiles(int pos0, int T) { return (pos0 + T + kKT - 1) / kKT; }
-int64_t attn_prefill_image_floats(int NKV, int pos0, int T) {
-    return static_cast<int64_t>(NKV) * attn_prefill_image_tiles(pos0, T) * kImgTile * 4;
-}
-
-int64_t attn_prefill_part_floats(int slots) { return static_cast<int64_t>(slots) * 16 * (kHD + 2); }
-int64_t attn_prefill_part_room(int64_t floats) {
-    return std::min<int64_t>(std::max<int64_t>(floats, 0) / (16 * (kHD + 2)), kFlashSlots);
+void attn_prefill_carve(AttnPrefillArgs& a, float* ws, int64_t floats) {
+    a.Qa = ws;
+    const int64_t used = attn_prefill_workspace_floats(a.NQ, a.T);
+    const AttnRoom r = attn_prefill_room(a.T, a.NQ, a.NKV, a.pos0, a.kv_bf16, device_cu_count(), floats - used);
+    ws += used;
+    if (r.image) {
+        a.kv_img = ws;
+        ws += attn_prefill_image_floats(a.NKV, a.pos0, a.T);
+    }
+    a.plan = r.plan;
+    if (r.plan.pieces) {
+        a.part = ws;
+        a.part_ml = reinterpret_cast<float2*>(ws + static_cast<int64_t>(r.plan.slots) * 16 * kHD);
+    }
 }
 
 hipError_t launch_attn_prefill(const AttnPrefillArgs& in, hipStream_t s) {
@@ -1726,10 +1730,7 @@ hipError_t launch_attn_prefill(const AttnPrefillArgs& in, hipStream_t s) {
     else klaunch(attn_prefill_prep_any_kernel, dim3(a.T, a.NQ + a.NKV), 256, 0, s, a);
     const int waves = flash_waves(a.kv_bf16), kQT = 16 * waves;
     const int blocks = (a.T * (a.NQ / a.NKV) + kQT - 1) / kQT * a.NKV;
-    FlashPlan p{};
-    if (a.part) p = flash_plan(a.T, a.NQ, a.NKV, a.pos0, a.kv_bf16, device_cu_count(), a.part_slots);
-    a.piece = p.piece;
-    a.part_ml = p.pieces ? reinterpret_cast<float2*>(a.part + static_cast<int64_t>(p.slots) * 16 * kHD) : nullptr;
+    const FlashPlan& p = a.plan;
     const dim3 grid = p.pieces ? dim3(p.pieces, blocks) : dim3(blocks);
     const bool img = !a.kv_bf16 && a.kv_img;
     if (img) {

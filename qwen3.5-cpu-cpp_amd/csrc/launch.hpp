@@ -273,24 +273,18 @@ struct AttnPrefillArgs {
     const float* rope_cs;      // optional [max_ctx][ROT] cos | sin table (else computed)
     float* omax = nullptr;     // maximum |out| of each (token, head): [T][NQ] (may be null)
     int out_tiled = 0;         // out in the xt_off layout (K = NQ * HD)
-    // optional (fp32 cache): attn_prefill_image_floats(NKV, pos0, T) floats, 16-byte aligned,
-    // for the keys and values pre-split into the attention kernel's tile layout
+    // set by attn_prefill_carve: the keys and values pre-split into the attention kernel's tile
+    // layout (fp32 cache; null: every workgroup splits them), how the keys are cut, and the
+    // pieces' partial outputs with the (max, sum) of each slot's 16 rows
     void* kv_img = nullptr;
-    int img_tiles = 0;  // set by the launch
-    // optional: attn_prefill_part_floats(part_slots) floats, 16-byte aligned, for the partial
-    // outputs of key ranges (flash_plan, which cuts into at most part_slots; without them no
-    // block is split)
+    FlashPlan plan{};
     float* part = nullptr;
-    int part_slots = 0;
-    int piece = 0;               // set by the launch: tiles of 32 keys per workgroup
-    float2* part_ml = nullptr;   // set by the launch: (max, sum) of each slot's 16 rows
+    float2* part_ml = nullptr;
+    int img_tiles = 0;  // set by the launch
 };
-int64_t attn_prefill_part_floats(int slots);
-// slots that `floats` floats have room for
-int64_t attn_prefill_part_room(int64_t floats);
-int64_t attn_prefill_workspace_floats(int NQ, int T);
-int attn_prefill_image_tiles(int pos0, int T);
-int64_t attn_prefill_image_floats(int NKV, int pos0, int T);
+// Workspace pointers and plan (plans.hpp) for `floats` >= attn_prefill_workspace_floats(NQ, T)
+// floats at ws, 16-byte aligned; the sizes, heads and cache type of `a` are set.
+void attn_prefill_carve(AttnPrefillArgs& a, float* ws, int64_t floats);
 hipError_t launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t s);
 // h[t][i] = silu(gu[t][2i]) * gu[t][2i + 1] (gate / up columns interleaved)
 // hidden[t][:] = bf16 embed[ids[t]][:]

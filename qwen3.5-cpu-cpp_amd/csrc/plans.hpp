@@ -17,11 +17,12 @@ constexpr int kFlashSlots = 8192;   // most partial outputs ("slots": 16 rows of
 constexpr int kFlashWhole = 64;     // blocks of up to so many tiles are never cut
 
 // How the attention kernel splits a block of T tokens at pos0 over key ranges: tiles per piece,
-// pieces of the longest row block (0: not split), the slots that takes, and the expected time
-// (in tiles; 0 where no split is considered).
+// pieces of the longest row block (0: not split), the slots that takes, the expected time (in
+// tiles; 0 where no split is considered), and the same were all pieces as long as the longest
+// (whole rounds of workgroups).
 struct FlashPlan {
     int piece, pieces, slots;
-    double time;
+    double time, rounds;
 };
 
 // Cuts blocks into pieces where the longest block would outlast an even share of the work, into
@@ -44,12 +45,13 @@ inline FlashPlan flash_plan(int T, int NQ, int NKV, int pos0, bool kv_bf16, int 
     const auto tiles = [&](int64_t b) {
         return static_cast<int>((pos0 + std::min<int64_t>(rows - 1, b * kQT + kQT - 1) / grp) / kKT + 1);
     };
-    FlashPlan p{0, 0, 0, 0.0};
+    FlashPlan p{0, 0, 0, 0.0, 0.0};
     const int most = tiles(nblk - 1);
     if (most <= kFlashWhole || items >= 2 * cu) return p;
     const auto ranked = [&](int64_t r) { return r < items ? tiles(nblk - 1 - r / NKV) : 0; };
     p.time = most;
     for (int i = 0; i < cu && cu + i < items; ++i) p.time = std::max<double>(p.time, ranked(cu - 1 - i) + ranked(cu + i));
+    p.rounds = p.time;
     double best = 0.9 * p.time;
     for (int pieces = 2; pieces <= kFlashPieces && pieces * items * waves <= room; ++pieces) {
         const int c = (most + pieces - 1) / pieces;
@@ -61,10 +63,51 @@ inline FlashPlan flash_plan(int T, int NQ, int NKV, int pos0, bool kv_bf16, int 
         const double t = (n <= cu ? c + 1.0 : static_cast<double>(all + n) / cu + 0.6 * c) + 4.0 + 0.01 * n;
         if (t < best) {
             best = t;
-            p = FlashPlan{c, (most + c - 1) / c, static_cast<int>((most + c - 1) / c * items * waves), t};
+            p = FlashPlan{c, (most + c - 1) / c, static_cast<int>((most + c - 1) / c * items * waves), t,
+                          static_cast<double>((n + cu - 1) / cu * (c + 1))};
         }
     }
     return p;
+}
+
+// Workspace of the attention prefill in floats, all multiples of 16 bytes: the query rows; the
+// keys and values of positions [0, pos0 + T) of an fp32 cache pre-split into the kernel's tile
+// layout (K chunks [3 parts][2][32][16] of 16 bytes a tile, as many for V); the slots' partial
+// outputs with their rows' maxima and sums.
+constexpr int kImgK = 3 * 2 * 32 * 16;  // 16-byte chunks of a tile's K
+constexpr int kImgTile = 2 * kImgK;
+inline int64_t attn_prefill_workspace_floats(int NQ, int T) { return static_cast<int64_t>(NQ) * T * 256 + 64; }
+inline int attn_prefill_image_tiles(int pos0, int T) {
+    return static_cast<int>((static_cast<int64_t>(pos0) + T + kKT - 1) / kKT);
+}
+inline int64_t attn_prefill_image_floats(int NKV, int pos0, int T) {
+    return static_cast<int64_t>(NKV) * attn_prefill_image_tiles(pos0, T) * kImgTile * 4;
+}
+inline int64_t attn_prefill_part_floats(int64_t slots) { return slots * 16 * (256 + 2); }
+
+// What the attention prefill does with `floats` of workspace beyond its query rows: the tile
+// image, then partial outputs in the rest, or without the image more of those. The image comes
+// first unless that costs the cut more than it saves (1.05 to 1.2 of a cut block's time from 300
+// tokens on, 1.25 to 1.3 of an uncut one's). Which cut is the faster one is told by the rounds:
+// over 454 pairs of cuts (64 to 2000 tokens, 16 / 2 and 8 / 2 heads, 2100 to 32000 positions,
+// rooms between) the choice was never more than 0.4% slower than without the image and 0.7%
+// slower than the faster of the two on average; 700 tokens of 16 heads, 16000 positions: image
+// and 5632 slots 955 us against 1115 with 7744 slots alone; 1200 at 2100: image and 2400 slots
+// 492, 3600 slots alone 427.
+struct AttnRoom {
+    bool image;
+    FlashPlan plan;
+};
+constexpr double kImageGain = 1.15;
+inline AttnRoom attn_prefill_room(int T, int NQ, int NKV, int pos0, bool kv_bf16, int n_cu, int64_t floats) {
+    const auto plan = [&](int64_t room) {
+        return flash_plan(T, NQ, NKV, pos0, kv_bf16, n_cu, std::max<int64_t>(room, 0) / attn_prefill_part_floats(1));
+    };
+    const AttnRoom without{false, plan(floats)};
+    const int64_t img = attn_prefill_image_floats(NKV, pos0, T);
+    if (kv_bf16 || img > floats) return without;
+    const AttnRoom with{true, plan(floats - img)};
+    return with.plan.rounds <= kImageGain * without.plan.rounds ? with : without;
 }
 
 }  // namespace q35k

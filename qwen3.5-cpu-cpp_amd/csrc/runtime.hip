@@ -1200,17 +1200,7 @@ q35_status prefill_block(q35_model* m, const PrefillPlan& p, int pos0, int T, in
             a.v_cache = kv_ptr(m, ly.idx, 1, 0);
             a.kv_bf16 = m->kv_elem == 2;
             a.rope_cs = m->rope_cs;
-            a.Qa = ws;
-            // the partial outputs of split key ranges (few tokens over many keys), then the
-            // pre-split key / value tiles where they fit in the rest of the workspace (the GDN
-            // layers' share is the larger one at 2B shapes: up to ~35k keys)
-            int64_t used = q35k::attn_prefill_workspace_floats(NQ, T);
-            a.part_slots = q35k::flash_plan(T, NQ, NKV, pos0, a.kv_bf16, m->n_cu, q35k::attn_prefill_part_room(p.ws_n - used)).slots;
-            if (a.part_slots) {
-                a.part = ws + used;
-                used += q35k::attn_prefill_part_floats(a.part_slots);
-            }
-            if (!a.kv_bf16 && used + q35k::attn_prefill_image_floats(NKV, pos0, T) <= p.ws_n) a.kv_img = ws + used;
+            q35k::attn_prefill_carve(a, ws, p.ws_n);
             a.out = mix;
             a.omax = mix_max;
             a.out_tiled = p.tiled;

@@ -2,11 +2,22 @@
 #include "plans.hpp"
 
 extern "C" {
-void flash_plan_c(int T, int NQ, int NKV, int pos0, int kv_bf16, int n_cu, int64_t room, int* out, double* time) {
+void flash_plan_c(int T, int NQ, int NKV, int pos0, int kv_bf16, int n_cu, int64_t room, int* out, double* time,
+                  double* rounds) {
     const q35k::FlashPlan p = q35k::flash_plan(T, NQ, NKV, pos0, kv_bf16 != 0, n_cu, room);
     out[0] = p.piece;
     out[1] = p.pieces;
     out[2] = p.slots;
     *time = p.time;
+    *rounds = p.rounds;
+}
+// out: image, piece, pieces, slots
+void attn_room_c(int T, int NQ, int NKV, int pos0, int kv_bf16, int n_cu, int64_t floats, int* out, double* rounds) {
+    const q35k::AttnRoom r = q35k::attn_prefill_room(T, NQ, NKV, pos0, kv_bf16 != 0, n_cu, floats);
+    out[0] = r.image;
+    out[1] = r.plan.piece;
+    out[2] = r.plan.pieces;
+    out[3] = r.plan.slots;
+    *rounds = r.plan.rounds;
 }
 }

@@ -20,9 +20,9 @@ def lib(tmp_path_factory):
 
 
 def flash(lib, T, nq, nkv, pos0, bf16, room=FULL, cu=256):
-    out, t = (C.c_int * 3)(), C.c_double()
-    lib.flash_plan_c(T, nq, nkv, pos0, int(bf16), cu, C.c_int64(room), out, C.byref(t))
-    return out[0], out[1], out[2], t.value
+    out, t, r = (C.c_int * 3)(), C.c_double(), C.c_double()
+    lib.flash_plan_c(T, nq, nkv, pos0, int(bf16), cu, C.c_int64(room), out, C.byref(t), C.byref(r))
+    return out[0], out[1], out[2], t.value, r.value
 
 
 def test_key_ranges_fit_the_room_and_cover_the_keys(lib):
@@ -33,7 +33,7 @@ def test_key_ranges_fit_the_room_and_cover_the_keys(lib):
         rooms = sorted(rng.sample(range(FULL + 1), 3)) + [FULL]
         before = None
         for room in [0] + rooms:
-            piece, pieces, slots, t = flash(lib, T, nq, nkv, pos0, bf16, room)
+            piece, pieces, slots, t, _ = flash(lib, T, nq, nkv, pos0, bf16, room)
             waves = 4 if bf16 else 8
             blocks = -(-T * (nq // nkv) // (16 * waves)) * nkv
             tiles = (pos0 + T - 1) // 32 + 1
@@ -54,9 +54,53 @@ def test_less_room_still_cuts(lib, nq, bf16):
     dropped = 0.0
     for pos0 in (2100, 4000, 8000, 16000, 32000):
         for T in range(20, 2049, 20):
-            _, _, slots, t = flash(lib, T, nq, 2, pos0, bf16)
+            _, _, slots, t, _ = flash(lib, T, nq, 2, pos0, bf16)
             half = flash(lib, T, nq, 2, pos0, bf16, FULL // 2)[3]
             assert half <= 1.3 * t, (T, pos0)
             if slots > FULL // 2:
                 dropped = max(dropped, flash(lib, T, nq, 2, pos0, bf16, 0)[3] / t)
     assert dropped > 1.5
+
+
+def image_floats(nkv, pos0, T):
+    return nkv * -(-(pos0 + T) // 32) * 32 * 768  # 3 KB per position and head
+
+
+def room(lib, T, nq, nkv, pos0, bf16, floats, cu=256):
+    out, t = (C.c_int * 4)(), C.c_double()
+    lib.attn_room_c(T, nq, nkv, pos0, int(bf16), cu, C.c_int64(floats), out, C.byref(t))
+    return out[0], out[3], t.value
+
+
+def test_image_and_partial_outputs_share_the_room(lib):
+    """Both where both fit; the image where it fits unless cutting without it is expected to gain
+    more; never past the room; nothing of it for a bf16 cache."""
+    rng = random.Random(11)
+    for _ in range(2000):
+        nq, nkv = rng.choice([(16, 2), (8, 2), (4, 1), (2, 1), (4, 4)])
+        T, pos0 = int(2 ** rng.uniform(0, 12)), rng.choice([0, int(2 ** rng.uniform(5, 16))])
+        img = image_floats(nkv, pos0, T)
+        _, _, slots, _, t = flash(lib, T, nq, nkv, pos0, False)
+        assert room(lib, T, nq, nkv, pos0, False, img + slots * 4128) == (1, slots, t)
+        assert room(lib, T, nq, nkv, pos0, True, 1 << 40)[:2] == (0, flash(lib, T, nq, nkv, pos0, True)[2])
+        floats = int(rng.uniform(0, 1.2) * (img + slots * 4128))
+        image, used, got = room(lib, T, nq, nkv, pos0, False, floats)
+        assert image * img + used * 4128 <= floats
+        alone = flash(lib, T, nq, nkv, pos0, False, floats // 4128)[4]
+        if image:
+            assert got <= 1.15 * alone
+        else:
+            assert got == alone
+            if img <= floats:
+                assert flash(lib, T, nq, nkv, pos0, False, (floats - img) // 4128)[4] > 1.15 * alone
+
+
+def test_image_is_kept_beside_a_smaller_cut(lib):
+    """16 / 2 heads, 54.6M floats less the query rows (the prompt arena's of 4096-token blocks of
+    the 2B shape): turns for which both do not fit keep the image with a smaller cut where that
+    measured faster, and leave it where it did not."""
+    for T, pos0, keep in ((520, 18000, 1), (700, 16000, 1), (1200, 20000, 1), (700, 20000, 0), (520, 16000, 0)):
+        floats = 54_600_000 - 16 * T * 256
+        assert image_floats(2, pos0, T) + 4128 * flash(lib, T, 16, 2, pos0, False)[2] > floats
+        image, slots, _ = room(lib, T, 16, 2, pos0, False, floats)
+        assert image == keep and slots
