@@ -87,18 +87,19 @@ inline int64_t attn_prefill_part_floats(int64_t slots) { return slots * 16 * (25
 
 // What the attention prefill does with `floats` of workspace beyond its query rows: the tile
 // image, then partial outputs in the rest, or without the image more of those. The image comes
-// first unless that costs the cut more than it saves (1.05 to 1.2 of a cut block's time from 300
-// tokens on, 1.25 to 1.3 of an uncut one's). Which cut is the faster one is told by the rounds:
-// over 454 pairs of cuts (64 to 2000 tokens, 16 / 2 and 8 / 2 heads, 2100 to 32000 positions,
-// rooms between) the choice was never more than 0.4% slower than without the image and 0.7%
-// slower than the faster of the two on average; 700 tokens of 16 heads, 16000 positions: image
-// and 5632 slots 955 us against 1115 with 7744 slots alone; 1200 at 2100: image and 2400 slots
-// 492, 3600 slots alone 427.
+// first unless that costs the cut more than it saves, and it saves what its readers, the row
+// blocks of a head, would spend on splitting the tiles themselves: 5 to 20% of a cut of many
+// blocks, 25 to 30% of uncut ones, nothing where fewer than 8 blocks read it. Which of two cuts is
+// the faster one is told by their rounds. Over 1106 pairs (16 to 2000 tokens, 16 / 2 and 8 / 2
+// heads, 2100 to 32000 positions, rooms between) the choice was within 2% of the one without the
+// image or faster in all but two (7%), and on average 0.8% slower than the faster of the two: 700
+// tokens of 16 heads at 16000 positions, image and 5632 slots 955 us against 1115 with 7744 slots
+// alone; 1200 at 2100, image and 2400 slots 492, 3600 slots alone 427; 1500 at 8000, image and
+// no cut 1263, 7520 slots alone 1399.
 struct AttnRoom {
     bool image;
     FlashPlan plan;
 };
-constexpr double kImageGain = 1.15;
 inline AttnRoom attn_prefill_room(int T, int NQ, int NKV, int pos0, bool kv_bf16, int n_cu, int64_t floats) {
     const auto plan = [&](int64_t room) {
         return flash_plan(T, NQ, NKV, pos0, kv_bf16, n_cu, std::max<int64_t>(room, 0) / attn_prefill_part_floats(1));
@@ -107,7 +108,21 @@ inline AttnRoom attn_prefill_room(int T, int NQ, int NKV, int pos0, bool kv_bf16
     const int64_t img = attn_prefill_image_floats(NKV, pos0, T);
     if (kv_bf16 || img > floats) return without;
     const AttnRoom with{true, plan(floats - img)};
-    return with.plan.rounds <= kImageGain * without.plan.rounds ? with : without;
+    const int64_t blocks = (static_cast<int64_t>(T) * (NQ / NKV) + 16 * flash_waves(false) - 1) / (16 * flash_waves(false));
+    const double gain = !with.plan.pieces ? 1.35 : blocks >= 8 ? 1.15 : 1.0;
+    return with.plan.rounds <= gain * without.plan.rounds ? with : without;
+}
+
+// Slots a program that keeps one workspace for all blocks of up to T tokens within max_ctx
+// positions sets aside: none where nothing is ever cut, no more than the most pieces of every
+// row block, and at most half of kFlashSlots (68 MB; a cut into those is at most 1.3 times the
+// time of the best one by the estimate above). Never less for more tokens or positions.
+inline int attn_prefill_share_slots(int T, int NQ, int NKV, bool kv_bf16, int64_t max_ctx) {
+    if (max_ctx <= kFlashWhole * kKT) return 0;
+    const int waves = flash_waves(kv_bf16), kQT = 16 * waves;
+    const int64_t items = (static_cast<int64_t>(T) * (NQ / NKV) + kQT - 1) / kQT * NKV;
+    const int64_t pieces = std::min<int64_t>(kFlashPieces, (max_ctx + kKT - 1) / kKT);
+    return static_cast<int>(std::min<int64_t>(items * waves * pieces, kFlashSlots / 2));
 }
 
 }  // namespace q35k

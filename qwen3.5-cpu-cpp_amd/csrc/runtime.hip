@@ -122,9 +122,13 @@ struct q35_model {
 
     // prompt arena: token-block activations of the chunked prefill (one hipMalloc), planned
     // at creation for blocks of up to pf_planned tokens, or made by the first prefill when
-    // none was planned (and made again only for a larger block)
+    // none was planned (and made again only for a larger block, or where a grown context gives
+    // the attention key ranges to cut)
     uint8_t* pf_arena = nullptr;
     size_t pf_bytes = 0;
+    int64_t pf_ws_end = 0;  // end of the mixers' workspace in the arena (floats)
+    int pf_tokens = 0;      // tokens of a block and attention partial outputs (slots) it was made for
+    int pf_share = 0;
     int pf_block = 0;    // requested block size (0 = automatic)
     int pf_planned = 0;  // block size planned at creation (0: none)
     int pf_exact = 0;    // prefill GEMMs on three exact bf16 parts (no fp16 weight copies)
@@ -718,7 +722,10 @@ struct PrefillPlan {
     int tb = 0, lr = 0;  // tokens per block, logits rows per output-head pass
     int tiled = 0;       // xn, mix, hb in the tiled layout of the two-part GEMM (H, I % 32 == 0)
     int64_t hidden = 0, xn = 0, proj = 0, mix = 0, hb = 0, ws = 0, logits = 0, ids = 0, total = 0;
-    int64_t ws_n = 0;  // floats at ws
+    // floats at ws: what the mixers (and the logits) need, and with room for the attention's tile
+    // image or the outputs of its cut (`share` slots)
+    int64_t ws_need = 0, ws_n = 0;
+    int share = 0;
     // row maxima of the GEMM inputs (xn, mix, hb), the weight maxima, the fp16 weights
     int64_t xn_max = 0, mix_max = 0, hb_max = 0, wmax = 0, wh = 0;
 };
@@ -741,7 +748,8 @@ int64_t proj_width(const q35_dims& d) {
                              2LL * d.attn_q_heads * d.attn_head_dim + 2LL * d.attn_kv_heads * d.attn_head_dim);
 }
 
-PrefillPlan plan_prefill(const q35_dims& d, int tb, int64_t logits_width, bool exact) {
+// max_ctx: positions a block may reach (0: not known yet, taken as many).
+PrefillPlan plan_prefill(const q35_dims& d, int tb, int64_t logits_width, bool exact, int64_t max_ctx, bool kv_bf16) {
     PrefillPlan p;
     p.tb = tb;
     p.lr = std::min(tb, 256);
@@ -761,19 +769,25 @@ PrefillPlan plan_prefill(const q35_dims& d, int tb, int64_t logits_width, bool e
     p.proj = take(T * proj_width(d));
     p.mix = take(TP * std::max(VD, QD));
     p.hb = take(TP * I);
-    // (the attention's share has room for half of the largest split of its key ranges, 66 MB:
-    // what a few tokens on a long context need; at 4096 tokens the GDN share is the larger one)
-    p.ws_n = std::max(q35k::gdn_prefill_workspace_floats(d.gdn_k_heads, d.gdn_v_heads, tb),
-                      q35k::attn_prefill_workspace_floats(d.attn_q_heads, tb) +
-                          q35k::attn_prefill_part_floats(q35k::kFlashSlots / 2));
-    p.ws = take(p.ws_n);
-    p.logits = take(static_cast<int64_t>(p.lr) * logits_width);
     p.ids = take(T);
     p.xn_max = take(T);
     p.mix_max = take(T * std::max(d.attn_q_heads, d.gdn_v_heads));
     p.hb_max = take(std::max(T * q35k::gemm_col_tiles(2 * d.ffn_intermediate),
                              std::min<int64_t>(T, q35k::kGemmSmallRows) * q35k::gemm_small_max_parts(2 * d.ffn_intermediate)));
     p.wmax = take(4LL * d.n_layers_total);
+    // the mixers' workspace, last before the weights: smaller blocks leave it more. The logits lie
+    // in it too (the output head runs after the last layer's mixer). An fp32 cache's blocks that are
+    // never cut have room for their tile image there, longer contexts for the cut's outputs
+    const int64_t qa = q35k::attn_prefill_workspace_floats(d.attn_q_heads, tb);
+    const int64_t ctx = max_ctx > 0 ? max_ctx : int64_t{1} << 30;
+    p.share = q35k::attn_prefill_share_slots(tb, d.attn_q_heads, d.attn_kv_heads, kv_bf16, ctx);
+    const int64_t img = kv_bf16 ? 0 : q35k::attn_prefill_image_floats(
+        d.attn_kv_heads, 0, static_cast<int>(std::min<int64_t>(ctx, q35k::kFlashWhole * q35k::kKT)));
+    p.ws_need = std::max({q35k::gdn_prefill_workspace_floats(d.gdn_k_heads, d.gdn_v_heads, tb), qa,
+                          static_cast<int64_t>(p.lr) * logits_width});
+    p.ws_n = std::max({p.ws_need, qa + img, qa + q35k::attn_prefill_part_floats(p.share)});
+    p.ws = p.logits = cur;
+    take(p.ws_n);
     if (p.tiled) {  // the fp16 weight copies of the two-part path
         int64_t wh = 0;
         for (int l = 0; l < d.n_layers_total; ++l) {
@@ -789,9 +803,11 @@ PrefillPlan plan_prefill(const q35_dims& d, int tb, int64_t logits_width, bool e
 
 int64_t logits_width(const q35_model* m) { return std::max<int64_t>(m->d.vocab_size, m->embed_rows); }
 
-size_t prompt_arena_bytes(const q35_model* m, int64_t tb) {
-    return static_cast<size_t>(plan_prefill(m->d, static_cast<int>(tb), logits_width(m), m->pf_exact).total) * 4;
+PrefillPlan plan_prefill(const q35_model* m, int64_t tb) {
+    return plan_prefill(m->d, static_cast<int>(tb), logits_width(m), m->pf_exact, m->max_ctx, m->kv_elem == 2);
 }
+
+size_t prompt_arena_bytes(const q35_model* m, int64_t tb) { return static_cast<size_t>(plan_prefill(m, tb).total) * 4; }
 
 // The prefill's fp16 weight copies, in the prompt arena: per matrix its maximum |w| (one
 // readback for all), then wh = fp16(w x 2^e) with e = 15 - (exponent of the maximum as in
@@ -830,20 +846,29 @@ q35_status make_prefill_weights(q35_model* m, const PrefillPlan& p) {
     return Q35_OK;
 }
 
-q35_status make_prompt_arena(q35_model* m, int64_t tb) {
+// The arena for blocks of tb tokens in place of the model's (freed first, unless the old one is
+// to stay where the device has no room for the new one beside it).
+q35_status make_prompt_arena(q35_model* m, int64_t tb, bool keep_old = false) {
+    const PrefillPlan plan = plan_prefill(m, tb);
+    const size_t bytes = static_cast<size_t>(plan.total) * 4;
+    void* p = nullptr;
+    if (keep_old && dev_alloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return Q35_OK;
+    }
     if (m->pf_arena) {
         HIPCHK(hipStreamSynchronize(m->stream));
         HIPCHK(hipFree(m->pf_arena));
         m->pf_arena = nullptr;
         m->pf_bytes = 0;
     }
-    void* p = nullptr;
-    const size_t bytes = prompt_arena_bytes(m, tb);
-    HIPCHK(dev_alloc(&p, bytes));
+    if (!p) HIPCHK(dev_alloc(&p, bytes));
     m->pf_arena = static_cast<uint8_t*>(p);
     m->pf_bytes = bytes;
+    m->pf_ws_end = plan.tiled ? plan.wh : plan.total;
+    m->pf_tokens = plan.tb;
+    m->pf_share = plan.share;
     m->budget.prompt_arena_bytes = bytes;
-    const PrefillPlan plan = plan_prefill(m->d, static_cast<int>(tb), logits_width(m), m->pf_exact);
     return plan.tiled ? make_prefill_weights(m, plan) : Q35_OK;
 }
 
@@ -853,18 +878,25 @@ int prefill_block_tokens(const q35_model* m) {
 }
 
 // The prompt arena for the current block size: the one planned at creation, or the one the
-// last prefill made when it is large enough, else a new one (lazy mode only).
+// last prefill made when it is large enough, else a new one (lazy mode only). The plan's
+// workspace is all that the arena has.
 q35_status ensure_prefill_arena(q35_model* m, PrefillPlan* plan) {
     const int tb = prefill_block_tokens(m);
-    *plan = plan_prefill(m->d, tb, logits_width(m), m->pf_exact);
-    if (m->pf_arena && static_cast<size_t>(plan->total) * 4 <= m->pf_bytes) return Q35_OK;
+    *plan = plan_prefill(m, tb);
+    const int64_t room = m->pf_arena ? m->pf_ws_end - plan->ws : 0;
+    if (tb <= m->pf_tokens && room >= plan->ws_need &&
+        (m->pf_planned > 0 || room >= plan->ws_n || plan->share <= m->pf_share)) {
+        plan->ws_n = room;
+        return Q35_OK;
+    }
     if (m->pf_planned > 0)
         return q35::fail(Q35_ERR_RANGE, "a prefill block of %d tokens exceeds the prompt arena planned for %d", tb,
                          m->pf_planned);
-    const q35_status st = make_prompt_arena(m, tb);
-    if (st == Q35_OK)
-        std::cerr << "[q35] prompt arena: " << (m->pf_bytes >> 20) << " MiB for blocks of " << tb << " tokens\n";
-    return st;
+    const q35_status st = make_prompt_arena(m, std::max(tb, m->pf_tokens));
+    if (st != Q35_OK) return st;
+    plan->ws_n = m->pf_ws_end - plan->ws;
+    std::cerr << "[q35] prompt arena: " << (m->pf_bytes >> 20) << " MiB for blocks of " << m->pf_tokens << " tokens\n";
+    return Q35_OK;
 }
 
 q35_status create_model(const q35_dims* dims, const q35_tensor* ts, int nt, int64_t max_ctx, int kv_elem,
@@ -1694,6 +1726,11 @@ q35_status q35_model_reserve_context(q35_model* m, int64_t max_context) {
     // made the old arenas again): the model is reset
     HIPCHK(q35k::launch_fill_f32(m->state_arena, static_cast<int64_t>(m->state_bytes / 4), 0.0f, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
+    // a planned prompt arena gets room to cut the attention's keys once they are long enough
+    if (st == Q35_OK && m->pf_planned > 0 && m->pf_arena) {
+        const PrefillPlan plan = plan_prefill(m, m->pf_planned);
+        if (plan.share > m->pf_share && plan.ws + plan.ws_n > m->pf_ws_end) return make_prompt_arena(m, m->pf_planned, true);
+    }
     return st;
 }
 

@@ -20,4 +20,7 @@ void attn_room_c(int T, int NQ, int NKV, int pos0, int kv_bf16, int n_cu, int64_
     out[3] = r.plan.slots;
     *rounds = r.plan.rounds;
 }
+int share_slots_c(int T, int NQ, int NKV, int kv_bf16, int64_t max_ctx) {
+    return q35k::attn_prefill_share_slots(T, NQ, NKV, kv_bf16 != 0, max_ctx);
+}
 }
