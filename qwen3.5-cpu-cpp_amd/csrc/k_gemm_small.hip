@@ -35,21 +35,10 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-enum Path : int { kBf16 = 0, kF16 = 1, kF16Planes = 2 };  // X row-major / tiled (xt_off) / split (xp_off)
-
 constexpr int kStep = 32;             // k per matrix instruction
 constexpr int kSteps = 16;            // steps per partial sum
 constexpr int kBlk = kStep * kSteps;  // K of one partial sum (512, as k_gemm.hip)
-
-constexpr int kXcds = 8;              // XCDs: workgroups are dispatched to them in turn
-
-constexpr int max_waves(int mr, int nr) { return mr * nr <= 3 ? 12 : mr * nr <= 6 ? 8 : 4; }
-
-// How the matrix is cut: row tiles of whole 16-row blocks (at most mr of them), column tiles
-// of whole units of `unit` columns (at most 16 nr columns), both as even as they come.
-struct SmallPlan {
-    int mr, nr, rt, ct, unit;
-};
+static_assert(kBlk == kSmallBlk, "the plan's block of K");
 
 template <int PATH>
 using operand = typename std::conditional<PATH == kBf16, bf16x8, halfx8>::type;
@@ -342,59 +331,13 @@ hipError_t launch_path(const GemmArgs& a, const SmallPlan& p, hipStream_t s) {
         default: return hipErrorInvalidValue;
     }
 }
-constexpr int kTiles[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 5}, {2, 2}, {2, 3}, {2, 4}, {2, 5}, {3, 3}, {3, 5}, {4, 3}, {4, 4}};
 
 int path_of(const GemmArgs& a) {  // as launch_gemm's
     return a.Wh && a.xmax && a.xmax_n > 0 && a.x_tiled ? (a.x_planes ? kF16Planes : kF16) : kBf16;
 }
 
-// The tile with the least expected time, or false where the 128 x 128 tiles are expected to
-// be faster. The expected times are least-squares fits, in us, of this kernel's times over
-// 96 products of 1 to 768 tokens (all twelve tiles, the six projection shapes of the 0.8B
-// and 2B models, 10% rms): a launch, and for each 512-deep block of K the X and W lines of
-// all tiles on the busiest compute unit, and the products and the split of X of its busiest
-// SIMD. The tile so chosen took on average 1.2% longer than the best of the twelve. The
-// 128 x 128 kernel takes one time per tile alone on a compute unit and one per two that
-// share it (128 tokens by 8224 x 2048: 65 tiles 53 us, 512 tokens: 260 tiles 82 us).
 bool small_plan(const GemmArgs& a, SmallPlan* best) {
-    if (a.M > kGemmSmallRows) return false;  // from there on 128 x 128 tiles fill the chip for every N >= 2048
-    // us per 512-deep block: X (16 rows), W (16 columns), products (16 x 16 block), split (16 rows)
-    constexpr double kCost[3][4] = {{0.60, 0.43, 0.43, 0.43}, {0.42, 0.38, 0.41, 0.0}, {0.10, 0.41, 0.39, 0.21}};
-    constexpr double kBig[3][2] = {{12.2, 20.5}, {10.2, 16.0}, {8.0, 12.7}};  // one tile, two tiles per CU
-    constexpr double kLaunch = 4.5;
-    const int path = path_of(a), cu = std::max(kXcds, device_cu_count());
-    const int nblk = (a.K + kBlk - 1) / kBlk, blocks = (a.M + 15) / 16;
-    const int per_cu = (((a.N + 127) / 128) * ((a.M + 127) / 128) + cu - 1) / cu;
-    double least = 0.97 * (kLaunch + nblk * (kBig[path][0] * (per_cu & 1) + kBig[path][1] * (per_cu >> 1)));
-    bool found = false;
-    for (const auto& t : kTiles) {
-        const int mr = t[0], nr = t[1];
-        if (mr > blocks) continue;
-        SmallPlan p{mr, nr, (blocks + mr - 1) / mr, (a.N + 16 * nr - 1) / (16 * nr), a.N % 4 == 0 ? 4 : a.swiglu ? 2 : 1};
-        // workgroups of the busiest compute unit, and as many column tiles as that allows
-        // (rt > 1: whole columns of row tiles per XCD)
-        int k;
-        if (p.rt == 1) {
-            k = (p.ct + cu - 1) / cu;
-            p.ct = cu * k;
-        } else {
-            const int cux = cu / kXcds, c8 = (p.ct + kXcds - 1) / kXcds;
-            k = (c8 * p.rt + cux - 1) / cux;
-            p.ct = std::max(c8, cux * k / p.rt) * kXcds;
-        }
-        p.ct = std::min(p.ct, (a.N + p.unit - 1) / p.unit);
-        const int mw = max_waves(mr, nr), rounds = (nblk + mw - 1) / mw;
-        const int simd = std::max((k * nblk + 3) / 4, rounds);  // K blocks of the busiest SIMD
-        const double* c = kCost[path];
-        const double us = kLaunch + k * nblk * (c[0] * ((blocks + p.rt - 1) / p.rt) + c[1] * a.N / (16.0 * p.ct)) +
-                          simd * mr * (c[2] * nr + c[3]);
-        if (us < least) {
-            least = us;
-            *best = p;
-            found = true;
-        }
-    }
-    return found;
+    return gemm_small_plan(a.M, a.N, a.K, a.swiglu != 0, path_of(a), device_cu_count(), best);
 }
 
 }  // namespace

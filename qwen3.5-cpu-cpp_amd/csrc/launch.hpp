@@ -114,11 +114,9 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s);
 // The same results by the kernel for few tokens where it is expected to be faster (false: it
 // is not, nothing was launched). Called by launch_gemm, which has checked `a`.
 bool launch_gemm_small(const GemmArgs& a, hipStream_t s, hipError_t* e);
-// Partial maxima per row that launch_gemm(a) writes to a.ymax (a.ymax itself is not read),
-// and the most there can be for N columns of up to kGemmSmallRows rows
+// Partial maxima per row that launch_gemm(a) writes to a.ymax (a.ymax itself is not read); at
+// most gemm_small_max_parts(N) for up to kGemmSmallRows rows, else gemm_col_tiles(N)
 int gemm_ymax_parts(const GemmArgs& a);
-constexpr int kGemmSmallRows = 1024;
-inline int gemm_small_max_parts(int N) { return N / 16 + 272; }
 // Tiled activation layout of the two-part GEMM's X operand: blocks of 16 rows x 32 k
 // (512 floats), row block after row block and within one the k blocks in order; inside a
 // block [h][r][g][e] for k = 8 g + 4 h + e of row r: the 16 bytes a lane of the matrix-core

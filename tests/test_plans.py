@@ -118,3 +118,29 @@ def test_share_of_a_kept_workspace(lib):
         t = rng.randint(1, T)
         if t <= ctx:
             assert flash(lib, t, nq, nkv, rng.randint(0, ctx - t), bf16, FULL // 2)[2] <= n
+
+
+# ----------------------------------------------------------------------- few-token GEMM
+def small(lib, M, N, K, path, swiglu=False, cu=256):
+    out = (C.c_int * 5)()
+    return list(out) if lib.gemm_small_plan_c(M, N, K, int(swiglu), path, cu, out) else None
+
+
+def test_few_token_gemm_plans(lib):
+    """Every plan's tiles cover the product and hold no more than their form; its column tiles are
+    within what a caller sets aside for their row maxima, on any number of compute units."""
+    rng = random.Random(2)
+    for _ in range(20000):
+        swiglu = rng.random() < 0.5
+        M, N, K = int(2 ** rng.uniform(0, 10.2)), int(2 ** rng.uniform(1, 15)), 8 * int(2 ** rng.uniform(0, 11))
+        N += N % 2 if swiglu else 0
+        cu = rng.choice([1, 7, 32, 64, 128, 256, 256, 256, 304, 512, 1024])
+        p = small(lib, M, N, K, rng.randrange(3), swiglu, cu)
+        if p is None:
+            continue
+        mr, nr, rt, ct, unit = p
+        units, blocks = -(-N // unit), -(-M // 16)
+        assert M <= 1024 and 1 <= ct <= units and 1 <= rt <= blocks
+        assert unit % 2 == 0 or not swiglu
+        assert -(-units // ct) * unit <= 16 * nr and -(-blocks // rt) <= mr
+        assert ct <= lib.gemm_small_max_parts_c(N)
