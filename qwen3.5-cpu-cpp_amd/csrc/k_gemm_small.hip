@@ -307,7 +307,7 @@ template <int PATH, int MR, int NR>
 hipError_t launch_tile(const GemmArgs& a, const SmallPlan& p, hipStream_t s) {
     const int nblk = (a.K + kBlk - 1) / kBlk, mw = max_waves(MR, NR);
     const int rounds = (nblk + mw - 1) / mw, waves = (nblk + rounds - 1) / rounds;
-    const uint32_t lds = static_cast<uint32_t>(waves) * MR * NR * 64 * 16;  // at most 60 KB
+    const uint32_t lds = static_cast<uint32_t>(waves) * MR * NR * 64 * 16;  // at most 64 KB, (4, 4); 0.5 KB more are static
     const int grid = p.rt > 1 ? (p.ct + kXcds - 1) / kXcds * kXcds * p.rt : p.ct;
     klaunch(gemm_small_kernel<PATH, MR, NR>, dim3(grid), 64 * waves, lds, s, a, p);
     return hipGetLastError();

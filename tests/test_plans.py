@@ -144,3 +144,13 @@ def test_few_token_gemm_plans(lib):
         assert unit % 2 == 0 or not swiglu
         assert -(-units // ct) * unit <= 16 * nr and -(-blocks // rt) <= mr
         assert ct <= lib.gemm_small_max_parts_c(N)
+
+
+def test_the_tile_tests_reach_every_form(lib):
+    from test_gpu_gemm_few_tokens_tiles import SIZES
+    for f16, forms in SIZES.items():
+        assert len(forms) == 12
+        for form, sizes in forms.items():
+            for s in sizes:
+                assert tuple(small(lib, *s, path=int(f16))[:2]) == form, s
+    assert small(lib, 1025, 1024, 2048, 0) is None
