@@ -146,9 +146,14 @@ constexpr int kSmallTiles[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 5}, {2, 2}, {2, 3}
 // 96 products of 1 to 768 tokens (all twelve tiles, the six projection shapes of the 0.8B
 // and 2B models, 10% rms): a launch, and for each 512-deep block of K the X and W lines of
 // all tiles on the busiest compute unit, and the products and the split of X of its busiest
-// SIMD. The tile so chosen took on average 1.2% longer than the best of the twelve. The
-// 128 x 128 kernel takes one time per tile alone on a compute unit and one per two that
-// share it (128 tokens by 8224 x 2048: 65 tiles 53 us, 512 tokens: 260 tiles 82 us).
+// SIMD. Coefficients of the fit, not costs one by one: X and its split both grow with the row
+// blocks, which the fit cannot tell apart (it charges the split where X is already split, and not
+// where the fp16 path splits it). The tile so chosen took on average 1.2% longer than the best of
+// the twelve. The 128 x 128 kernel takes one time per tile alone on a compute unit and one per two
+// that share it (128 tokens by 8224 x 2048: 65 tiles 53 us, 512 tokens: 260 tiles 82 us). It stays
+// within 3% of its expected time, but with X as fp32 for the fp16 path and one or two blocks of K
+// (below the fitted products) within 10%: 256 tokens by 7168 x 1024, 0.93 expected, took 6 us more
+// than its 25, 384 by 5120 x 1024, 0.94, 3 us; at 0.9 and below at most 1.5 us, mostly less.
 inline bool gemm_small_plan(int M, int N, int K, bool swiglu, int path, int n_cu, SmallPlan* best) {
     if (M > kGemmSmallRows) return false;  // from there on 128 x 128 tiles fill the chip for every N >= 2048
     // us per 512-deep block: X (16 rows), W (16 columns), products (16 x 16 block), split (16 rows)
@@ -158,7 +163,7 @@ inline bool gemm_small_plan(int M, int N, int K, bool swiglu, int path, int n_cu
     const int cu = std::min(std::max(kXcds, n_cu), kSmallCus);
     const int nblk = (K + kSmallBlk - 1) / kSmallBlk, blocks = (M + 15) / 16;
     const int per_cu = (((N + 127) / 128) * ((M + 127) / 128) + cu - 1) / cu;
-    double least = 0.97 * (kLaunch + nblk * (kBig[path][0] * (per_cu & 1) + kBig[path][1] * (per_cu >> 1)));
+    double least = (path == kF16 && nblk <= 2 ? 0.90 : 0.97) * (kLaunch + nblk * (kBig[path][0] * (per_cu & 1) + kBig[path][1] * (per_cu >> 1)));
     bool found = false;
     for (const auto& t : kSmallTiles) {
         const int mr = t[0], nr = t[1];

@@ -154,3 +154,9 @@ def test_the_tile_tests_reach_every_form(lib):
             for s in sizes:
                 assert tuple(small(lib, *s, path=int(f16))[:2]) == form, s
     assert small(lib, 1025, 1024, 2048, 0) is None
+
+
+def test_shallow_products_with_the_fp16_split_leave_close_calls_to_the_tiles(lib):
+    for M, N, K in ((256, 7168, 1024), (384, 5120, 1024), (300, 6144, 1024)):
+        assert small(lib, M, N, K, 1) is None
+    assert small(lib, 192, 5120, 1024, 1) and small(lib, 900, 2048, 2048, 1)
