@@ -368,7 +368,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs a) {
 
 }  // namespace
 
-// Few tokens go to k_gemm_small.hip where that is expected to be faster (its small_plan).
+// Few tokens go to k_gemm_small.hip where that is expected to be faster (gemm_small_plan in plans.hpp).
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
     dim3 grid(gemm_col_tiles(a.N), (a.M + kBM - 1) / kBM);
     const bool f16 = a.Wh && a.xmax && a.xmax_n > 0 && a.x_tiled && a.K % 32 == 0;

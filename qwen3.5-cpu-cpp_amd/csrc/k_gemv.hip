@@ -502,12 +502,15 @@ hipError_t launch_kc(const GemvArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Widths of the models (1024 and 3584 of the 0.8B shape, 2048, 4096 and 6144) get compile-time
-// chunk counts: every chunk of a row group in flight at once, the input staged through registers
-// before them. Other widths up to 2048 stage through registers with chunks counted at run time
-// (the SwiGLU prologue, whose input is twice as wide, and other wider inputs stage through LDS
-// directly). Against that, 1024 and 3584: 2048 x 3584 5.3 -> 4.3 us, 16384 x 3584 20.7 -> 18.1,
-// 17 decode steps of the 0.8B shape 12.2 -> 9.8 ms.
+// Widths that the models' layers have (hidden and FFN sizes of the 0.8B and 2B shapes, and the 2B
+// shape's heads: 1024, 2048, 3584, 4096 and 6144, whole numbers of 512-wide chunks) get
+// compile-time chunk counts: every chunk of a row group in flight at once, the input staged
+// through registers before them. Other such widths could have them too, at a set of kernels each
+// (prologues, epilogues, rows per wave); none is used, so none is built. Other widths up to 2048
+// stage through registers with chunks counted at run time (the SwiGLU prologue, whose input is
+// twice as wide, and other wider inputs stage through LDS directly). Against that, 1024 and 3584:
+// 2048 x 3584 5.3 -> 4.3 us, 16384 x 3584 20.7 -> 18.1, 17 decode steps of the 0.8B shape 12.2 ->
+// 9.8 ms.
 template <int PRO, int EPI>
 hipError_t launch_rpw(const GemvArgs& a, hipStream_t s) {
     const bool gated_ok = PRO != kProGatedNorm || a.head_dim == 128;

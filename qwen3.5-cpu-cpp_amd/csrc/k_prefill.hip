@@ -993,20 +993,20 @@ constexpr float kLog2e = 1.44269504088896341f;
 
 // 128 query rows per workgroup (16 per wave), causal, keys of earlier blocks from the cache,
 // 32-key tiles staged through LDS (the next tile's rows are loaded into registers while the
-// current one is multiplied), online softmax. One workgroup per CU (112 KB of LDS with three
-// parts). A row is a (token, query head of the kv head's group) pair, row = token * group +
+// current one is multiplied), online softmax. One workgroup per CU (96 KB of LDS with three
+// parts; a bf16 cache's 4-wave workgroups hold 32 KB, two per CU). A row is a (token, query head of the kv head's group) pair, row = token * group +
 // head: the heads of a group read the same keys, so 32 tokens of a group of 4 are one full
 // block and not four quarter ones, and a block's rows end within 128 / group tokens of each
 // other. Causal work grows with the block, and workgroups are dispatched in linear order, so
 // rank L takes the L-th longest block of all kv heads.
 //
-// Few blocks over many keys (a chat turn: 300 tokens of 2 x 4 heads are 20 blocks) would
-// leave most compute units idle, so a block's tiles are then cut into pieces of `piece`
-// tiles, one workgroup each (flash_plan), whose unnormalised outputs, maxima and sums
-// flash_combine_kernel merges. 300 tokens at 7000 cached bf16 positions, 8 / 2 heads: 24
-// blocks of single heads 703 us; 494 pieces 82 us (flash 74, of which about 8 the query rows
-// and the partial outputs; merge 12 for 32 MB of them). Bound as the unsplit kernel: products
-// behind LDS reads and two barriers a tile.
+// Few blocks over many keys (a chat turn: 300 tokens of 2 x 4 heads are 20 blocks, 38 of a bf16
+// cache's 64 rows) would leave most compute units idle, so a block's tiles are then cut into
+// pieces of `piece` tiles, one workgroup each (flash_plan), whose unnormalised outputs, maxima
+// and sums flash_combine_kernel merges. That turn at 7000 cached bf16 positions: 703 us as 24
+// blocks of 128 tokens of single heads, 81 as 494 pieces (traced one by one: query rows 6, flash
+// 75, merge of 32 MB of partial outputs 12). Bound as the unsplit kernel: products behind LDS
+// reads and two barriers a tile.
 // Both products run on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16): every fp32 operand
 // is the exact sum of three bf16 parts (hi + mid + lo, as in the bf16 path of the projection GEMM), and a
 // product a.b is the sum of the six part products a_i b_j with i + j <= 2 (parts counted

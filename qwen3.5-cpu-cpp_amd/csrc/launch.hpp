@@ -284,7 +284,6 @@ struct AttnPrefillArgs {
 // floats at ws, 16-byte aligned; the sizes, heads and cache type of `a` are set.
 void attn_prefill_carve(AttnPrefillArgs& a, float* ws, int64_t floats);
 hipError_t launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t s);
-// h[t][i] = silu(gu[t][2i]) * gu[t][2i + 1] (gate / up columns interleaved)
 // hidden[t][:] = bf16 embed[ids[t]][:]
 hipError_t launch_embed_rows(const uint16_t* embed, const int* ids, float* hidden, int T, int H, hipStream_t s);
 

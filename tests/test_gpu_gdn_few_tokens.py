@@ -1,8 +1,8 @@
 """GDN prefill of few tokens (one launch, token by token) against the oracle's sequential
 recurrence at the bars of the other GDN prefill tests: one token, less than a conv run and one
-more, the largest block and one past it (the chunked kernels), positions that move the ring's
-slots, continuing, v-heads = 2 k-heads, the raw readout, and a state off its 16-byte alignment
-(chunked kernels, the same result within the bar)."""
+more, positions that move the ring's slots, continuing, v-heads = 2 k-heads, the raw readout, and
+a state off its 16-byte alignment (chunked kernels, the same result within the bar); 47, 48 and 49
+tokens run the chunked kernels (the 36-token limit of the one launch: test_gpu_gdn_edges.py)."""
 import ctypes as C
 
 import numpy as np
