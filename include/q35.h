@@ -204,7 +204,9 @@ q35_status q35_model_extend(q35_model *m, const int32_t *ids, int32_t n, float *
 /* Tokens per prefill block (0 = automatic: the planned block, else min(4096, max_context)).
  * Larger blocks make larger GEMMs and a larger prompt arena; a prompt arena planned at
  * creation serves every block up to its size and refuses larger ones (Q35_ERR_RANGE), one
- * made by a prefill is made again only for a larger block. */
+ * made by a prefill is made again only for a larger block. Past 2048 positions it also holds
+ * partial outputs of the attention (up to 68 MB): a context that grows past that makes it again,
+ * a planned one in q35_model_reserve_context where there is room beside the old one. */
 q35_status q35_model_set_prefill_block(q35_model *m, int32_t tokens);
 /* Output head of the prefill logits: Q35_HEAD_OUTPUT (the default) is the step's head
  * (lm_head when the checkpoint has one, else the tied embedding; vocab_size rows),
