@@ -861,6 +861,7 @@ q35_status make_prompt_arena(q35_model* m, int64_t tb, bool keep_old = false) {
         HIPCHK(hipFree(m->pf_arena));
         m->pf_arena = nullptr;
         m->pf_bytes = 0;
+        m->pf_tokens = m->pf_share = 0;
     }
     if (!p) HIPCHK(dev_alloc(&p, bytes));
     m->pf_arena = static_cast<uint8_t*>(p);
