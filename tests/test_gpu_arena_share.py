@@ -51,3 +51,23 @@ def test_room_after_the_context_grows(model_dirs, planned):
     fresh.close()
     np.testing.assert_array_equal(got, ref)
     assert rel_l2(got, ref) < REL_L2
+
+
+@pytest.mark.parametrize("kv", [4, 2])
+@pytest.mark.parametrize("T", [700, 1500])
+def test_long_turn_on_a_long_context(tmp_path, T, kv):
+    """16 / 2 heads at 8000 positions, a turn in one block whose best cut (more than 5000 slots) is
+    larger than the 4096 that the arena sets aside, against decoding it token by token."""
+    d = pyq35.dims_for("tiny")
+    d.n_layers_total, d.attn_interval, d.attn_q_heads, d.attn_kv_heads = 2, 2, 16, 2
+    pyq35.synth_write_model(str(tmp_path), d, seed=3, std=0.02)
+    ids = pyq35.synth_token_ids(11, d.vocab_size, T)
+    logits = []
+    for block in (T, 0):
+        m = pyq35.Model(str(tmp_path), 8000 + T, kv_bytes_per_elem=kv, prefill_block=block)
+        m.fill_synthetic(8000, seed=9)
+        logits.append(m.extend(ids)[0] if block else np.stack([m.step(int(i))[0] for i in ids]))
+        m.close()
+    # a bf16 row may round the other way: the bar of the bf16-cache model tests
+    bar = REL_L2 if kv == 4 else 2e-4
+    assert max(rel_l2(a, b) for a, b in zip(*logits)) < bar
